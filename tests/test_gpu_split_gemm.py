@@ -1,0 +1,145 @@
+"""The products that run on the bf16 matrix cores with their float32 operands
+split in three: sizes at the edges of its tiles and of the rules that pick it,
+and values the split cannot carry (infinities, NaN, sums that overflow)."""
+
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    from ttrl_amd.engine.device import open_device
+
+    return open_device(0)
+
+
+def _patches(x, k, s):
+    """(B, H, W, C) -> (B * OH * OW, k * k * C) in float64, k order (kh, kw, c)."""
+    oh = (x.shape[1] - k) // s + 1
+    ow = (x.shape[2] - k) // s + 1
+    cols = [x[:, i:i + s * oh:s, j:j + s * ow:s] for i in range(k) for j in range(k)]
+    return np.stack(cols, 3).reshape(x.shape[0] * oh * ow, -1).astype(np.float64)
+
+
+def _scatter(cols, shape, k, s):
+    """The adjoint of _patches: columns added back onto an image batch."""
+    b, h, w, c = shape
+    oh, ow = (h - k) // s + 1, (w - k) // s + 1
+    cols = cols.reshape(b, oh, ow, k * k, c)
+    out = np.zeros(shape)
+    for i in range(k):
+        for j in range(k):
+            out[:, i:i + s * oh:s, j:j + s * ow:s] += cols[:, :, :, i * k + j]
+    return out
+
+
+def _bound(terms, magnitude):
+    """Rounding of a float32 sum of `terms` products in any order: terms + 16
+    roundings (the split's dropped parts and the epilogue among the 16) of at
+    most 2^-24 of the sum of magnitudes."""
+    return (terms + 16) * 2.0 ** -24 * magnitude
+
+
+def _backward(dev, x, dy, wt, k, s, u8, scale=1.0, mask=None, bank=None):
+    """-> (dW, db, dX or None) of the convolution; with `bank`, the weight
+    gradient's partials formed by the launch that reads gradient banks."""
+    from ttrl_amd import _lib
+    from ttrl_amd.engine.tensor import DeviceArray, to_device
+
+    B = x.shape[0]
+    c, h, w = (x.shape[1], x.shape[2], x.shape[3]) if u8 else (x.shape[3], x.shape[1], x.shape[2])
+    o = dy.shape[1]
+    geom = _lib.ConvGeom(B, c, h, w, o, k, s, 0, _lib.LAYOUT_NCHW_U8 if u8 else _lib.LAYOUT_NHWC_F32)
+    xd, dyd = to_device(x, dev, x.dtype), to_device(dy, dev)
+    dw, db = DeviceArray(dev, (c * k * k, o)), DeviceArray(dev, (1, o))
+    if u8:
+        dev.call("ttrl_conv2d_backward_weight", C.byref(geom), xd.vp, C.c_float(scale), dyd.vp, None, dw.vp, db.vp,
+                 C.c_float(0.0))
+        return dw.numpy(), db.numpy(), None
+    wd, dx = to_device(wt, dev), DeviceArray(dev, x.shape)
+    md = None if mask is None else to_device(mask, dev)
+    mp = None if md is None else md.vp
+    if bank is None:
+        dev.call("ttrl_conv2d_backward", C.byref(geom), xd.vp, C.c_float(scale), dyd.vp, None, wd.vp, dw.vp, db.vp,
+                 C.c_float(0.0), dx.vp, mp, C.c_float(0.0))
+    else:
+        src = _lib.GradSource()
+        dev.call("ttrl_conv2d_backward_deferred", C.byref(geom), xd.vp, C.c_float(scale), dyd.vp, None, wd.vp, dw.vp,
+                 db.vp, dx.vp, mp, C.c_float(0.0), bank, C.byref(src))
+        assert src.kind == _lib.GRAD_SPLITS and src.splits > 1
+        dev.call("ttrl_grad_sources_materialize", 1, C.byref(src))
+    return dw.numpy(), db.numpy(), dx.numpy()
+
+
+# (batch, channels, size, out, kernel, stride): batches on both sides of each
+# rule's line, rows and columns one past a tile, input channels that are and
+# are not whole fragments of columns, strides whose residue classes differ.
+CONVS = [(166, 32, 8, 64, 3, 1), (167, 32, 8, 64, 3, 1), (400, 32, 7, 32, 2, 1), (251, 36, 9, 96, 5, 1),
+         (110, 32, 20, 64, 4, 2), (700, 64, 5, 32, 3, 1), (170, 20, 14, 64, 2, 2), (130, 96, 11, 20, 3, 1)]
+
+
+@pytest.mark.parametrize("b,c,size,o,k,s", CONVS)
+@pytest.mark.parametrize("bank", [None, 1])
+def test_convolution_gradients(dev, b, c, size, o, k, s, bank):
+    rng = np.random.default_rng(b)
+    x = rng.standard_normal((b, size, size, c)).astype(np.float32)
+    wt = rng.standard_normal((k * k * c, o)).astype(np.float32)
+    a = _patches(x, k, s)
+    dy = rng.standard_normal((a.shape[0], o)).astype(np.float32)
+    mask = x if bank is None else None
+    dw, db, dx = _backward(dev, x, dy, wt, k, s, False, 0.5, mask, bank)
+    g = dy.astype(np.float64)
+    assert np.all(np.abs(dw - 0.5 * (a.T @ g)) <= _bound(a.shape[0], np.abs(a).T @ np.abs(g)))
+    assert np.all(np.abs(db[0] - g.sum(0)) <= _bound(a.shape[0], np.abs(g).sum(0)))
+    w64 = wt.astype(np.float64)
+    want = 0.5 * _scatter(g @ w64.T, x.shape, k, s)
+    magnitude = _scatter(np.abs(g) @ np.abs(w64).T, x.shape, k, s)
+    if mask is not None:
+        want = np.where(mask > 0, want, 0.0)
+    assert np.all(np.abs(dx - want) <= _bound(k * k * o, magnitude))
+
+
+@pytest.mark.parametrize("b,c,h,w,o", [(15, 4, 84, 84, 32), (16, 4, 84, 84, 32), (25, 3, 100, 100, 16), (700, 1, 36, 36, 32),
+                                       (90, 4, 84, 52, 20), (97, 2, 84, 84, 64)])
+def test_frames_weight_gradient(dev, b, c, h, w, o):
+    rng = np.random.default_rng(b)
+    x = rng.integers(0, 256, (b, c, h, w), dtype=np.uint8)
+    a = _patches(x.transpose(0, 2, 3, 1), 8, 4).reshape(-1, 64, c).transpose(0, 2, 1).reshape(-1, c * 64)
+    dy = rng.standard_normal((a.shape[0], o)).astype(np.float32)
+    dw, db, _ = _backward(dev, x, dy, None, 8, 4, True, 1.0 / 255.0)
+    g = dy.astype(np.float64)
+    scale = np.float64(np.float32(1.0 / 255.0))
+    assert np.all(np.abs(dw - scale * (a.T @ g)) <= scale * _bound(a.shape[0], np.abs(a).T @ np.abs(g)))
+    assert np.all(np.abs(db[0] - g.sum(0)) <= _bound(a.shape[0], np.abs(g).sum(0)))
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3.3e38, 1e-38])
+def test_values_outside_the_split(dev, value):
+    """A value bf16 parts cannot carry gives what float32 gives in the sums
+    that read it, and leaves the others alone."""
+    rng = np.random.default_rng(3)
+    x = rng.standard_normal((200, 9, 9, 32)).astype(np.float32)
+    x[..., 5] = 1.0  # no lower parts: inf * 0 must not appear
+    wt = rng.uniform(0.25, 0.5, (9 * 32, 64)).astype(np.float32)
+    a = _patches(x, 3, 1)
+    dy = rng.standard_normal((a.shape[0], 64)).astype(np.float32)
+    dy[1234, 7] = value
+    dw, db, dx = _backward(dev, x, dy, wt, 3, 1, False)
+    g, w64 = dy.astype(np.float64), wt.astype(np.float64)
+    with np.errstate(all="ignore"):
+        wants = ((dw, a.T @ g, a.shape[0], np.abs(a).T @ np.abs(g)),
+                 (db[0], g.sum(0), a.shape[0], np.abs(g).sum(0)),
+                 (dx, _scatter(g @ w64.T, x.shape, 3, 1), 9 * 64, _scatter(np.abs(g) @ w64.T, x.shape, 3, 1)))
+        for got, want, terms, magnitude in wants:
+            bad = ~np.isfinite(want.astype(np.float32))
+            assert np.array_equal(np.isnan(got[bad]), np.isnan(want[bad]))
+            some = bad & ~np.isnan(want)
+            assert np.array_equal(np.sign(got[some]), np.sign(want[some]))
+            fine = ~bad & (magnitude < 1e38)
+            assert np.all(np.abs(got - want)[fine] <= _bound(terms, magnitude[fine]))

@@ -425,13 +425,16 @@ struct EpConvDx {
     FDiv d_nhnw, d_nw;
     float alpha, beta;
   };
-  template <class F>
-  __device__ __forceinline__ void with_bound(int grp, F&& f) const {
+  __device__ __forceinline__ Bound bound(int grp) const {
     const Params q = pin_pod(Params{dx, xmask, uint32_t(long(g.B) * g.H * g.W * g.C * 4), rows(grp), g.C, g.H, g.W,
                                     g.S, g.nw[grp], g.ih0[grp], g.iw0[grp], g.d_nhnw[grp], g.d_nw[grp], alpha, beta});
-    f(Bound{q.rows, q.C, q.H, q.W, q.S, q.nw, q.ih0, q.iw0, q.d_nhnw, q.d_nw, make_res(q.dx, q.bytes),
-            make_res(q.xm, q.xm ? q.bytes : 0u), make_res(q.dx, q.beta != 0.f ? q.bytes : 0u), q.xm != nullptr,
-            q.alpha, q.beta});
+    return Bound{q.rows, q.C, q.H, q.W, q.S, q.nw, q.ih0, q.iw0, q.d_nhnw, q.d_nw, make_res(q.dx, q.bytes),
+                 make_res(q.xm, q.xm ? q.bytes : 0u), make_res(q.dx, q.beta != 0.f ? q.bytes : 0u), q.xm != nullptr,
+                 q.alpha, q.beta};
+  }
+  template <class F>
+  __device__ __forceinline__ void with_bound(int grp, F&& f) const {
+    f(bound(grp));
   }
 };
 

@@ -9,7 +9,7 @@
 // (outside capture, on scratch outputs) and keep the faster for the context.
 //   dW = sum over taps of X-slice^T dY  ttrl/engine/conv/backward.py:45-78
 //   dX = conv_transpose2d(dY, W)        ttrl/engine/conv/backward.py:33-42
-#include "conv.hpp"
+#include "conv_split.hpp"
 
 namespace ttrl {
 namespace {
@@ -123,6 +123,23 @@ template <int MODE>
 int conv_backward_chosen(ttrl_ctx* ctx, const ConvGeo& g, const void* x, float x_scale, const float* dy,
                          const float* wt, float* dwt, float* db, float beta_w, float* dx, const float* xmask,
                          float beta_x, long reserved, float* bank = nullptr, ttrl_grad_source* out = nullptr) {
+  if constexpr (MODE != kPatchGeneral) {
+    // Both gradients on the split core, where it takes both: a launch each.
+    const ConvDxProblem d0 = conv_dx_problem(g, 0, dy, wt, dx, xmask, x_scale, beta_x);
+    int rc = TTRL_OK;
+    if (dx_split(g, d0).wm &&
+        conv_dw_split(ctx, conv_dw_problem<MODE>(g, x, x_scale, dy, dwt, db, beta_w), g, x, x_scale, dy, dwt, db,
+                      reserved, bank, out, "ttrl_conv2d_backward", &rc)) {
+      for (int c0 = 0; c0 < g.S * g.S && rc == TTRL_OK; c0 += kMaxGroups) {
+        const ConvDxProblem d = conv_dx_problem(g, c0, dy, wt, dx, xmask, x_scale, beta_x);
+        const SplitTile t = dx_split(g, d);
+        rc = t.wm ? run_dx_split(ctx, t, d, "ttrl_conv2d_backward")
+                  : run_gemm<kConvDxCfgs>(ctx, d.la, d.lb, d.ep, d.q.M, d.q.N, d.q.K, d.q.groups,
+                                          "ttrl_conv2d_backward", reserved);
+      }
+      return rc;
+    }
+  }
   if (pair_is_faster<MODE>(ctx, g, x, x_scale, dy, wt, xmask, reserved, bank))
     return conv_backward_pair<MODE>(ctx, g, x, x_scale, dy, wt, dwt, db, beta_w, dx, xmask, beta_x, reserved, bank,
                                     out);

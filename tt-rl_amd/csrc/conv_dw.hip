@@ -1,7 +1,7 @@
 // Convolution weight gradient: dW = sum over pixels of patch^T dZ, the bias
 // gradient folded in as an implicit ones row of the patch matrix.
 //   dW = sum over taps of X-slice^T dY  ttrl/engine/conv/backward.py:45-78
-#include "conv.hpp"
+#include "conv_split.hpp"
 
 namespace ttrl {
 namespace {
@@ -12,6 +12,11 @@ int conv_backward_weight_mode(ttrl_ctx* ctx, const ConvGeo& g, const void* x, fl
                               float* dwt, float* db, float beta, long reserved, float* bank = nullptr,
                               ttrl_grad_source* out = nullptr) {
   const ConvDwProblem<MODE> p = conv_dw_problem<MODE>(g, x, x_scale, dy, dwt, db, beta);
+  if constexpr (MODE != kPatchGeneral) {
+    int rc = TTRL_OK;
+    if (conv_dw_split(ctx, p, g, x, x_scale, dy, dwt, db, reserved, bank, out, "ttrl_conv2d_backward_weight", &rc))
+      return rc;
+  }
   if (!bank)
     return run_gemm<CFGS>(ctx, p.la, p.lb, p.ep, p.q.M, p.q.N, p.q.K, 1, "ttrl_conv2d_backward_weight", reserved);
   GemmPlan plan{};

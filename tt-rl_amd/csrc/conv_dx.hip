@@ -3,7 +3,7 @@
 // kernel taps, so each class is a plain GEMM and every dX element is
 // written exactly once (no atomics).
 //   dX = conv_transpose2d(dY, W)        ttrl/engine/conv/backward.py:33-42
-#include "conv.hpp"
+#include "conv_split.hpp"
 
 using namespace ttrl;
 
@@ -23,8 +23,12 @@ int ttrl_conv2d_backward_input(ttrl_ctx* ctx, const ttrl_conv_geom* geom, const 
   }
   for (int c0 = 0; c0 < g.S * g.S; c0 += kMaxGroups) {
     const ConvDxProblem p = conv_dx_problem(g, c0, dy, wt, dx, xmask, x_scale, beta);
-    rc = run_gemm<kConvDxCfgs>(ctx, p.la, p.lb, p.ep, p.q.M, p.q.N, p.q.K, p.q.groups, "ttrl_conv2d_backward_input",
-                               reserved);
+    const SplitTile t = dx_split(g, p);
+    if (t.wm)
+      rc = run_dx_split(ctx, t, p, "ttrl_conv2d_backward_input");
+    else
+      rc = run_gemm<kConvDxCfgs>(ctx, p.la, p.lb, p.ep, p.q.M, p.q.N, p.q.K, p.q.groups, "ttrl_conv2d_backward_input",
+                                 reserved);
     if (rc) return rc;
   }
   return TTRL_OK;

@@ -1,0 +1,237 @@
+// Convolution operands of the split-bf16 core (split_gemm.hpp).
+#pragma once
+
+#include "conv.hpp"
+#include "split_gemm.hpp"
+
+namespace ttrl {
+
+// Input-gradient A of a residue class (LdConvDxA): row r is an input pixel, k =
+// (jh, jw, o) with O a multiple of 32, so a step is 32 channels of one tap.
+struct SaConvDx {
+  LdConvDxA src;
+  using Params = LdConvDxA::Params;
+  struct Live {
+    static constexpr bool EXACT = false, PERM = true, TABLE = false;
+    Params q;
+    __amdgpu_buffer_rsrc_t rs;
+    struct Raw { f32x4 a, b; };
+    struct Row { uint32_t off; int ohc, owc; };
+    struct Kb { uint32_t off; int jh, jw; };
+    __device__ __forceinline__ Row row(int r, int lg) const {
+      const LdConvDxA::Live::Row x = LdConvDxA::Live{q, rs}.row(r);
+      return Row{uint32_t(x.base) * 4u + uint32_t(lg) * 16u, x.ohc, x.owc};
+    }
+    __device__ __forceinline__ Kb kbase(int k0) const {
+      const LdConvDxA::Live::Kp x = LdConvDxA::Live{q, rs}.kpos(__builtin_amdgcn_readfirstlane(k0));
+      return Kb{uint32_t(x.off) * 4u, x.v ? x.jh : 1 << 28, x.jw};
+    }
+    __device__ __forceinline__ void issue(const Row& r, const Kb& k, Raw& f) const {
+      const bool in = uint32_t(r.ohc - k.jh) < uint32_t(q.OH) && uint32_t(r.owc - k.jw) < uint32_t(q.OW);
+      const uint32_t o = in ? r.off + k.off : kBad;
+      f.a = ld_f4(rs, o);
+      f.b = ld_f4(rs, o + 64u);
+    }
+    __device__ __forceinline__ void resolve(const Raw& f, f32x4& a, f32x4& b) const {
+      a = f.a;
+      b = f.b;
+    }
+  };
+  __device__ __forceinline__ Live live(int grp) const {
+    const LdConvDxA::Live l = src.live(grp);
+    return Live{l.q, l.rs};
+  }
+};
+
+// Input-gradient B (LdConvDxB): column n = c, k contiguous along o.
+struct SbConvDx {
+  LdConvDxB src;
+  using Params = LdConvDxB::Params;
+  struct Live {
+    static constexpr bool COL = false;
+    Params q;
+    __amdgpu_buffer_rsrc_t rs;
+    __device__ __forceinline__ uint32_t row(int n) const { return n < q.C ? uint32_t(n * q.O) * 4u : kBad; }
+    __device__ __forceinline__ uint32_t kbase(int k0) const {
+      return LdConvDxB::Live{q, rs}.kpos(__builtin_amdgcn_readfirstlane(k0)).off;
+    }
+    __device__ __forceinline__ float elem(int n, int k) const {
+      return ld_f1(rs, row(n) + LdConvDxB::Live{q, rs}.kpos(k).off);
+    }
+  };
+  __device__ __forceinline__ Live live(int grp) const {
+    const LdConvDxB::Live l = src.live(grp);
+    return Live{l.q, l.rs};
+  }
+};
+
+// Input-gradient epilogue (EpConvDx); C a multiple of the columns a lane stores.
+struct SeConvDx {
+  EpConvDx src;
+  struct Bound {
+    EpConvDx::Bound b;
+    __amdgpu_buffer_rsrc_t rc, rm;
+    __device__ __forceinline__ uint32_t off(int r, int c) const {
+      const int n = b.d_nhnw.div(r);
+      const int rem = r - n * b.d_nhnw.d;
+      const int i = b.d_nw.div(rem), j = rem - i * b.nw;
+      const int ih = b.ih0 + b.S * i, iw = b.iw0 + b.S * j;
+      return r < b.rows && c < b.C ? uint32_t(((n * b.H + ih) * b.W + iw) * b.C + c) * 4u : kBad;
+    }
+    template <int FN>
+    __device__ __forceinline__ FVec<FN> bias(int) const { return FVec<FN>(0.f); }
+    __device__ __forceinline__ float alpha() const { return b.alpha; }
+    __device__ __forceinline__ float beta() const { return b.beta; }
+    __device__ __forceinline__ bool relu() const { return false; }
+    __device__ __forceinline__ bool masked() const { return b.has_xm; }
+    __device__ __forceinline__ bool accumulates() const { return b.beta != 0.f; }
+  };
+  __device__ __forceinline__ int rows(int grp) const { return src.rows(grp); }
+  __device__ __forceinline__ void store_sum(int, int, float) const {}
+  __device__ __forceinline__ Bound bind(int grp) const {
+    const EpConvDx::Bound b = src.bound(grp);
+    return Bound{b, b.rdx, b.rxm};
+  }
+};
+
+// Weight-gradient A(r = patch index, k = pixel): a lane's 8 k are 8 pixels,
+// whose byte offsets the workgroup tabulates; its row's offset in the patch
+// is its own.  Vector patch layouts only (no padding); uint8 frames are exact
+// in one bf16.
+template <bool U8>
+struct SaPatchT {
+  ConvGeo g;
+  const void* x;
+  uint32_t xbytes;
+
+  struct Params {
+    ConvCore g;
+    const void* x;
+    uint32_t xbytes;
+  };
+  struct Live {
+    static constexpr bool EXACT = U8, PERM = false, TABLE = true;
+    Params q;
+    __amdgpu_buffer_rsrc_t rs;
+    struct Raw { f32x4 a, b; };
+    using Row = uint32_t;
+    __device__ __forceinline__ uint32_t row(int r, int) const { return tap_off(q.g, r); }
+    __device__ __forceinline__ uint32_t offset(int m) const { return pixel_base(q.g, m); }
+    __device__ __forceinline__ float one(uint32_t o) const {
+      if constexpr (U8) return __uint_as_float(ld_u8(rs, o));
+      else return ld_f1(rs, o);
+    }
+    __device__ __forceinline__ void issue(uint32_t row, const u32x4& o0, const u32x4& o1, Raw& f) const {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        f.a[j] = one(row + o0[j]);
+        f.b[j] = one(row + o1[j]);
+      }
+    }
+    __device__ __forceinline__ void resolve(const Raw& f, f32x4& a, f32x4& b) const {
+      a = f.a;
+      b = f.b;
+      if constexpr (U8)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          a[j] = float(__float_as_uint(f.a[j]));
+          b[j] = float(__float_as_uint(f.b[j]));
+        }
+    }
+  };
+  __device__ __forceinline__ Live live(int) const {
+    const Params q = pin_pod(Params{conv_core(g), x, xbytes});
+    return Live{q, make_res(q.x, q.xbytes)};
+  }
+};
+
+inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+// How the split core runs a weight gradient: K (the pixels) in `splits` parts
+// of `kchunk`, as many as fill the device twice with 64-row tiles and as the
+// room for partials and kMaxDwSplits (whoever sums them reads them all)
+// allow.  splits 0: the FP32 core, for operands that do not fit (out channels
+// in whole float4s) and for fewer than kSplitPixels pixels, where a part is too
+// short to pay for more partials (third layer with its sum at 4,900 pixels:
+// FP32 13.7 us, split 15.0; at 6,272: 15.5 / 15.0).
+constexpr int kMaxDwSplits = 64;
+constexpr int kSplitPixels = 6000;
+struct DwSplit {
+  SplitTile tile;
+  int splits = 0, kchunk = 0;
+};
+inline DwSplit dw_split(const ConvGeo& g, const float* dy, int ones, long room) {
+  DwSplit d;
+  if (g.O % 4 || g.M < kSplitPixels || !aligned16(dy) || gemm_force_set()) return d;
+  const int kp = g.C * g.KH * g.KW;
+  d.tile = SplitTile{1, g.O > 32 ? 4 : 2};
+  const long tiles = long(ceil_div(kp, 64)) * ceil_div(g.O, 16 * d.tile.fn);
+  const long stages = ceil_div(g.M, kSplitKB);
+  const long most = std::min({room / (long(kp + ones) * g.O), long(kMaxDwSplits), stages});
+  const long want = std::min(most, std::max(2L, 512 / tiles));
+  if (want < 2 || want * tiles < 128) return d;
+  const long per = ceil_div(stages, want);
+  d.splits = int(ceil_div(stages, per));
+  d.kchunk = int(per) * kSplitKB;
+  return d;
+}
+
+// Its launch: partials [splits][kp + ones][O] to `part`.
+template <bool U8>
+inline int run_dw_split(ttrl_ctx* ctx, const DwSplit& d, const ConvGeo& g, const void* x, const float* dy, int ones,
+                        float* part, const char* name) {
+  const SaPatchT<U8> la{g, x, input_bytes(g)};
+  SbCol lb;  // B(k = m, n = o) = dZ[m][o]
+  lb.p[0] = dy;
+  lb.ld = lb.rows = g.O;
+  lb.K = g.M;
+  SeStore ep;  // the partials' reader applies the epilogue
+  ep.M = g.C * g.KH * g.KW;
+  ep.N = g.O;
+  return run_split(ctx, d.tile, la, lb, ep, ep.M, g.O, g.M, 1, name, ones, part, d.splits, d.kchunk);
+}
+
+// The weight gradient on the split core, if it takes it: its partials left in
+// `bank` and described by *out (bank not null), or summed from the workspace.
+template <int MODE>
+inline bool conv_dw_split(ttrl_ctx* ctx, const ConvDwProblem<MODE>& p, const ConvGeo& g, const void* x, float x_scale,
+                          const float* dy, float* dwt, float* db, long reserved, float* bank, ttrl_grad_source* out,
+                          const char* name, int* rc) {
+  long wsf = kGradBankFloats;
+  float* part = bank;
+  if (!part) {
+    part = ctx_workspace(ctx, &wsf);
+    wsf -= reserved;
+  }
+  const int ones = db ? 1 : 0;
+  const DwSplit d = dw_split(g, dy, ones, wsf);
+  if (!d.splits) return false;
+  *rc = run_dw_split<MODE == kPatchU8Word>(ctx, d, g, x, dy, ones, part, name);
+  if (*rc != TTRL_OK) return true;
+  if (bank) {
+    GemmPlan plan{};
+    plan.splits = d.splits;
+    *out = conv_dw_source(g, x_scale, dwt, db, part, plan);
+    return true;
+  }
+  FDiv dn;
+  dn.set(p.q.N);
+  const unsigned blocks = std::min(2048u, unsigned(long(p.q.M) * p.q.N / 256 + 1));
+  hipLaunchKernelGGL((k_splitk_reduce<EpStore>), dim3(blocks, 1), dim3(256), 0, stream_of(ctx), part, p.ep, p.q.M, p.q.N,
+                     d.splits, dn);
+  *rc = check_launch(name);
+  return true;
+}
+
+// Whether the split core runs the input gradient of the classes of `p`.
+inline SplitTile dx_split(const ConvGeo& g, const ConvDxProblem& p) {
+  if (g.O % 32 || g.C % 4 || gemm_force_set() || !aligned16(p.la.dy) || !aligned16(p.lb.wt) || !aligned16(p.ep.dx) ||
+      !aligned16(p.ep.xmask))
+    return SplitTile{};
+  return split_tile(p.q.M, p.q.N, p.q.groups);
+}
+inline int run_dx_split(ttrl_ctx* ctx, const SplitTile& t, const ConvDxProblem& p, const char* name) {
+  return run_split(ctx, t, SaConvDx{p.la}, SbConvDx{p.lb}, SeConvDx{p.ep}, p.q.M, p.q.N, p.q.K, p.q.groups, name);
+}
+
+}  // namespace ttrl

@@ -8,7 +8,7 @@
 //   relu / relu_bw        ttrl/engine/ops/unary.py:25-37
 //   bias-gradient sum     ttrl/engine/ops/broadcast.py:11-30
 //   log_std clamp         ttrl/nets/heads.py:65-93, ttrl/engine/ops/select.py:52-63
-#include "tile_gemm.hpp"
+#include "split_gemm.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -107,6 +107,21 @@ bool plan_valid(const GemmPlan& p, int M, int N, int K, int groups, long ws_floa
   const int spb = p.kchunk / t.tbk;
   if (p.splits != (stages + spb - 1) / spb) return false;  // the splits exactly cover K
   return p.splits == 1 || long(p.splits) * groups * M * N <= ws_floats;
+}
+
+SplitTile split_tile(long M, long N, long groups) {
+  SplitTile t;
+  t.fn = N > 32 ? 4 : 2;
+  const long cols = ceil_div(N, 16 * t.fn) * groups;
+  const long t64 = ceil_div(M, 64) * cols, t128 = ceil_div(M, 128) * cols;
+  if (t64 < kSplitTiles) return SplitTile{};
+  t.wm = double(ceil_div(t128, 256)) <= 0.55 * double(ceil_div(t64, 256)) ? 2 : 1;
+  return t;
+}
+
+bool gemm_force_set() {
+  const char* v = std::getenv("TTRL_GEMM_FORCE");
+  return v && *v;
 }
 
 bool gemm_forced(unsigned allowed, int M, int N, int K, int groups, long ws_floats, GemmPlan* out) {

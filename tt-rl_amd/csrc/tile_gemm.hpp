@@ -979,6 +979,7 @@ bool gemm_tuning_enabled();
 bool gemm_tuning_log();  // TTRL_GEMM_TUNE_LOG=1: print each tuned signature's candidates to stderr
 // TTRL_GEMM_FORCE="cfg[:splits]" (read on every call, for tests): run that
 // tile shape wherever a call site allows it, bypassing the plan cache.
+bool gemm_force_set();
 bool gemm_forced(unsigned allowed, int M, int N, int K, int groups, long ws_floats, GemmPlan* out);
 
 template <int ID_, int BM_, int BN_, int WGM_, int WGN_, int WGK_, int TBK_>
