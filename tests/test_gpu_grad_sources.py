@@ -406,3 +406,25 @@ def test_wide_outer_source_formed_by_tiles(device, rows, cols, batch):
     for k in ("p", "g", "S", "V", "step"):
         assert np.array_equal(got[k].numpy(), ref[k].numpy()), k
     assert got["gsq"].numpy()[0] == pytest.approx(float(ref["gsq"].numpy()[0]), rel=1e-5)
+
+
+@pytest.mark.parametrize("rows,cols,batch", [(100, 128, 33), (70, 64, 64), (33, 192, 75), (32, 64, 257)])
+def test_tiles_of_more_batch_rows_than_one_slice(device, rows, cols, batch):
+    """Tiles that stage the batch in several slices give the bits of the
+    element-by-element path, which a v off float4 alignment takes."""
+    from ttrl_amd import _lib
+
+    rng = np.random.default_rng(batch)
+    u = _up(device, rng.standard_normal((batch, rows)))
+    flat = rng.standard_normal(batch * cols)
+    v, off = _up(device, flat), _up(device, np.concatenate([[0.0], flat]))
+    out = []
+    for p in (v.ptr, off.ptr + 4):
+        g = _empty(device, (rows * cols + cols,))
+        src = (_lib.GradSource * 1)(_lib.GradSource(kind=_lib.GRAD_OUTER, rows=rows, cols=cols, dw=g.ptr,
+                                                    db=g.ptr + 4 * rows * cols, u=u.ptr, v=p, batch=batch))
+        device.call("ttrl_grad_sources_materialize", 1, src)
+        out.append(g.numpy())
+    assert np.array_equal(out[0], out[1])
+    want = u.numpy().astype(np.float64).T @ v.numpy().reshape(batch, cols).astype(np.float64)
+    assert _rel(out[0][:rows * cols], want.ravel()) < 1e-5

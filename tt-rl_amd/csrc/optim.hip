@@ -331,13 +331,15 @@ constexpr int kOuterLds = 2048;   // v floats an outer-product source stages in 
 constexpr int kOuterULds = 6144;  // u floats (the workgroup's slice of rows) it stages
 constexpr int kOuterChunk = 32;   // batch rows of u staged per memory round trip
 constexpr int kSumLds = 1024;    // terms of an ordered sum staged in LDS
-// A wide outer-product source (cols a multiple of kTileCols, batch <=
-// kTileBatch) is formed by tiles: one workgroup per kTileRows x kTileCols
-// block of the weight, kTileOuts float4s per thread (tile rows tr and
-// tr + 16 of one float4 column), its slices of u and v staged in LDS, so
-// each workgroup reads [batch][32] of u and [batch][64] of v however wide
-// the layer is, and a layer of 3136 x 512 takes 784 workgroups (one wave of
-// the chip's resident workgroups with the rest of the step).  The bias's
+// A wide outer-product source (cols a multiple of kTileCols) is formed by
+// tiles: one workgroup per kTileRows x kTileCols block of the weight,
+// kTileOuts float4s per thread (tile rows tr and tr + 16 of one float4
+// column), its slices of u and v staged in LDS kTileBatch batch rows at a
+// time, so each workgroup reads [batch][32] of u and [batch][64] of v however
+// wide the layer is, and a layer of 3136 x 512 takes 784 workgroups (one wave
+// of the chip's resident workgroups with the rest of the step).  The next
+// slice is loaded while this one's products run; past the first it is LDS
+// reads that bound it (MEASURED_TILE).  The bias's
 // gradient (sum_b v[b][c]) is formed by the first row band's tiles, from
 // the rows of v they have staged: lanes 0 .. kTileCols/4 - 1 of wave 0 take
 // one float4 of the tile's columns each.
@@ -517,25 +519,25 @@ __device__ __forceinline__ f32x4 outer_grad_staged(const GradSrc& s, const Outer
 }
 
 // A tile's slices: loaded into registers (issue_outer_tile), then written
-// to LDS (commit_outer_tile): us[b][i] = u[b][r0 + i] (rows past the block
-// repeat its last row, never used), vs[b][j] = v[b][c0 + j].  Work that does
+// to LDS (commit_outer_tile): us[b][i] = u[b0 + b][r0 + i] (rows past the block
+// repeat its last row, never used), vs[b][j] = v[b0 + b][c0 + j].  Work that does
 // not need them can run between the two while the loads are in flight.
 struct OuterTileLoads {
   float u[kTileBatch * kTileRows / kOptThreads];
   f32x4 v[kTileBatch * kTileCols / 4 / kOptThreads];
 };
-__device__ __forceinline__ OuterTileLoads issue_outer_tile(const GradSrc& s, int r0, int c0) {
+__device__ __forceinline__ OuterTileLoads issue_outer_tile(const GradSrc& s, int r0, int c0, int b0) {
   constexpr int NU = kTileBatch * kTileRows / kOptThreads, NV = kTileBatch * kTileCols / 4 / kOptThreads;
   const int tid = threadIdx.x;
   OuterTileLoads l;
 #pragma unroll
   for (int k = 0; k < NU; ++k) {
-    const int e = tid + k * kOptThreads, b = e / kTileRows, i = e - b * kTileRows;
+    const int e = tid + k * kOptThreads, i = e % kTileRows, b = b0 + e / kTileRows;
     l.u[k] = b < s.batch ? s.u[long(b) * s.rows + min(r0 + i, s.rows - 1)] : 0.f;
   }
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    const int e = tid + k * kOptThreads, b = e / (kTileCols / 4), j = e - b * (kTileCols / 4);
+    const int e = tid + k * kOptThreads, j = e % (kTileCols / 4), b = b0 + e / (kTileCols / 4);
     l.v[k] = b < s.batch ? *reinterpret_cast<const f32x4*>(s.v + long(b) * s.cols + c0 + 4 * j) : f32x4{};
   }
   return l;
@@ -550,16 +552,14 @@ __device__ __forceinline__ void commit_outer_tile(const OuterTileLoads& l, float
   __syncthreads();
 }
 // The thread's kTileOuts float4s (tile rows tr + kTileBand * o, float4
-// column tc4): the same sums in the same order as source_grad (b from zero,
-// fmaf(u, v, acc)).  The staged rows past the batch hold zeros, and adding
-// fmaf(0, 0, acc) = acc + 0 leaves acc's bits as they are (acc starts at +0
-// and a sum rounded to nearest is never -0 unless both terms are), so the
-// loop runs over all kTileBatch rows, unrolled by 8 (fully, its hoisted
-// reads would not fit the registers).
+// column tc4), the staged rows added: over all slices the same sums in the
+// same order as source_grad (b from zero, fmaf(u, v, acc)).  The staged rows
+// past the batch hold zeros, and adding fmaf(0, 0, acc) = acc + 0 leaves acc's
+// bits as they are (acc starts at +0 and a sum rounded to nearest is never -0
+// unless both terms are), so the loop runs over all kTileBatch rows, unrolled
+// by 8 (fully, its hoisted reads would not fit the registers).
 __device__ __forceinline__ void outer_grad_tile(const float* us, const float* vs, int tr, int tc4,
                                                 f32x4 (&acc)[kTileOuts]) {
-#pragma unroll
-  for (int o = 0; o < kTileOuts; ++o) acc[o] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 8
   for (int b = 0; b < kTileBatch; ++b) {
     const f32x4 v = reinterpret_cast<const f32x4*>(vs)[b * (kTileCols / 4) + tc4];
@@ -571,18 +571,16 @@ __device__ __forceinline__ void outer_grad_tile(const float* us, const float* vs
     }
   }
 }
-// The bias float4 of the tile's float4 column tc4: sum_b v[b][c] in the
-// order source_grad adds it (b from zero; the zero rows past the batch, as
-// above, change nothing).
-__device__ __forceinline__ f32x4 outer_bias_tile(const float* vs, int tc4) {
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+// The bias float4 of the tile's float4 column tc4, the staged rows added:
+// sum_b v[b][c] in the order source_grad adds it (b from zero; the zero rows
+// past the batch, as above, change nothing).
+__device__ __forceinline__ void outer_bias_tile(const float* vs, int tc4, f32x4& acc) {
 #pragma unroll 8
   for (int b = 0; b < kTileBatch; ++b) {
     const f32x4 v = reinterpret_cast<const f32x4*>(vs)[b * (kTileCols / 4) + tc4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[j] = fmaf(1.f, v[j], acc[j]);
   }
-  return acc;
 }
 // Where workgroup t of a tiled source works: its tile (the thread's float4
 // q[o] of the weight, ok[o] false past the block's rows) and, in the first
@@ -630,6 +628,25 @@ __device__ __forceinline__ TileSpot tile_spot(const GradSrc& s, int t) {
   o.bias_lane = o.bias_wave && tid < kTileCols / 4;
   o.qb = o.c0 / 4 + min(tid, kTileCols / 4 - 1);
   return o;
+}
+
+// A tile's gradients (and on its bias lanes the bias's) over the whole batch,
+// the first slice's loads given.
+__device__ __forceinline__ void outer_tile(const GradSrc& s, const TileSpot& t, OuterTileLoads& l, float* us, float* vs,
+                                           f32x4 (&gv)[kTileOuts], f32x4& gb) {
+#pragma unroll
+  for (int o = 0; o < kTileOuts; ++o) gv[o] = f32x4{0.f, 0.f, 0.f, 0.f};
+  gb = f32x4{0.f, 0.f, 0.f, 0.f};
+  commit_outer_tile(l, us, vs);
+  for (int b0 = kTileBatch;; b0 += kTileBatch) {
+    const bool more = b0 < s.batch;  // uniform
+    if (more) l = issue_outer_tile(s, t.r0, t.c0, b0);
+    outer_grad_tile(us, vs, t.tr, t.tc4, gv);
+    if (t.bias_lane) outer_bias_tile(vs, t.tc4, gb);
+    if (!more) return;
+    __syncthreads();
+    commit_outer_tile(l, us, vs);
+  }
 }
 
 // Ordered sums dst = scale * sum_{i<n} src[i*stride], one thread each.
@@ -736,7 +753,7 @@ __global__ __launch_bounds__(kOptThreads) __attribute__((amdgpu_waves_per_eu(4))
       // all in flight while the scalars are formed (unconditional, so that
       // thread 0's wait for the count waits for none of them; a row past the
       // block reads the block's first float4 and stores nothing)
-      const OuterTileLoads tl = issue_outer_tile(s, t.r0, t.c0);
+      OuterTileLoads tl = issue_outer_tile(s, t.r0, t.c0, 0);
       long i[kTileOuts];
       f32x4 pv[kTileOuts], sv[kTileOuts], vv[kTileOuts];
 #pragma unroll
@@ -757,9 +774,8 @@ __global__ __launch_bounds__(kOptThreads) __attribute__((amdgpu_waves_per_eu(4))
         vb = Vv[ib];
       }
       adam_scalars_of(stepc, a.lr, a.b1, a.b2, a.eps, &alpha_t, &eps_t);
-      commit_outer_tile(tl, us, vs);
-      f32x4 gv[kTileOuts];
-      outer_grad_tile(us, vs, t.tr, t.tc4, gv);
+      f32x4 gv[kTileOuts], gb;
+      outer_tile(s, t, tl, us, vs, gv, gb);
 #pragma unroll
       for (int o = 0; o < kTileOuts; ++o) {
         if (t.ok[o]) {
@@ -771,7 +787,6 @@ __global__ __launch_bounds__(kOptThreads) __attribute__((amdgpu_waves_per_eu(4))
         }
       }
       if (t.bias_lane) {
-        const f32x4 gb = outer_bias_tile(vs, t.tc4);
         if (STORE) Gd[ib] = gb;
         adam4(pb, gb, sb, vb, a.b1, a.b2, a.wd, eps_t, alpha_t, gsq);
         P[ib] = pb;
@@ -871,13 +886,13 @@ __global__ __launch_bounds__(kOptThreads) void k_sources_write(SrcSet a) {
   __shared__ float us[kOuterULds], vs[kOuterLds];
   if (s.tiled) {
     const TileSpot t = tile_spot(s, xcd_tile(blk, s.block0, s.blocks));
-    commit_outer_tile(issue_outer_tile(s, t.r0, t.c0), us, vs);
-    f32x4 gv[kTileOuts];
-    outer_grad_tile(us, vs, t.tr, t.tc4, gv);
+    OuterTileLoads tl = issue_outer_tile(s, t.r0, t.c0, 0);
+    f32x4 gv[kTileOuts], gb;
+    outer_tile(s, t, tl, us, vs, gv, gb);
 #pragma unroll
     for (int o = 0; o < kTileOuts; ++o)
       if (t.ok[o]) reinterpret_cast<f32x4*>(s.gw)[t.q[o]] = gv[o];
-    if (t.bias_lane) reinterpret_cast<f32x4*>(s.gb)[t.qb] = outer_bias_tile(vs, t.tc4);
+    if (t.bias_lane) reinterpret_cast<f32x4*>(s.gb)[t.qb] = gb;
     return;
   }
   const int qb0 = (blk - s.block0) * kOptThreads;
@@ -1049,7 +1064,7 @@ int make_sources(int n, const ttrl_grad_source* srcs, const float* g, long gn, G
       d.v = s.v;
       d.batch = s.batch;
       // wide enough that one row band of v would not fit in LDS: by tiles
-      d.tiled = s.cols % kTileCols == 0 && s.batch <= kTileBatch && aligned16(s.v) && s.batch * s.cols > kOuterLds;
+      d.tiled = s.cols % kTileCols == 0 && aligned16(s.v) && long(s.batch) * s.cols > kOuterLds;
       if (d.tiled) {
         d.ntc = s.cols / kTileCols;
         d.ntiles = int(ceil_div(long(s.rows), kTileRows)) * d.ntc;
