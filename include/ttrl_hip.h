@@ -244,6 +244,9 @@ int ttrl_linear_backward(ttrl_ctx* ctx, const ttrl_linear_desc* desc);
 
 #define TTRL_LAYOUT_NHWC_F32 0 /* [B][H][W][C] fp32 activations */
 #define TTRL_LAYOUT_NCHW_U8 1  /* [B][C][H][W] uint8 frames */
+/* Or-ed into in_layout: gradients summed by the FP32 matrix core alone, for
+ * callers whose next step turns a last-bit difference into a decision. */
+#define TTRL_CONV_FP32_ORDER 16
 
 /* Geometry of ConvGeometry (ttrl/engine/conv/geometry.py:94-199), square kernel. */
 typedef struct ttrl_conv_geom {

@@ -43,6 +43,7 @@ constexpr unsigned kConvGeneralCfgs = cfg_bit(T32x32) | cfg_bit(T64x32);
 
 struct ConvGeo {
   int B, C, H, W, O, KH, KW, S, P, OH, OW, u8;
+  int fp32_order;                  // TTRL_CONV_FP32_ORDER: not on the split core
   int M;                           // B * OH * OW
   FDiv d_ohow, d_ow, d_c, d_kw, d_khkw, d_o, d_tw, d_s;
   int TH, TW;                      // taps per class along h and w: ceil(K / S)
@@ -469,8 +470,9 @@ inline int make_geo(const ttrl_conv_geom* s, ConvGeo& g) {
   TTRL_REQUIRE(span_h % s->stride == 0 && span_w % s->stride == 0,
                "conv: ragged geometry (in %dx%d, k %d, s %d, p %d) leaves input rows that feed no output",
                s->in_h, s->in_w, s->kernel, s->stride, s->padding);
-  TTRL_REQUIRE(s->in_layout == TTRL_LAYOUT_NHWC_F32 || s->in_layout == TTRL_LAYOUT_NCHW_U8,
-               "conv: unknown input layout %d", s->in_layout);
+  const int layout = s->in_layout & ~TTRL_CONV_FP32_ORDER;
+  TTRL_REQUIRE(layout == TTRL_LAYOUT_NHWC_F32 || layout == TTRL_LAYOUT_NCHW_U8, "conv: unknown input layout %d",
+               s->in_layout);
   g.B = s->batch;
   g.C = s->in_c;
   g.H = s->in_h;
@@ -481,7 +483,8 @@ inline int make_geo(const ttrl_conv_geom* s, ConvGeo& g) {
   g.P = s->padding;
   g.OH = span_h / s->stride + 1;
   g.OW = span_w / s->stride + 1;
-  g.u8 = s->in_layout == TTRL_LAYOUT_NCHW_U8 ? 1 : 0;
+  g.u8 = layout == TTRL_LAYOUT_NCHW_U8 ? 1 : 0;
+  g.fp32_order = s->in_layout & TTRL_CONV_FP32_ORDER ? 1 : 0;
   g.M = g.B * g.OH * g.OW;
   // Buffer loads address operands with 32-bit byte offsets below 2^30.
   const long bigs[] = {long(g.B) * g.OH * g.OW * g.O * 4, long(g.B) * g.H * g.W * g.C * (g.u8 ? 1 : 4),

@@ -162,7 +162,7 @@ struct DwSplit {
 };
 inline DwSplit dw_split(const ConvGeo& g, const float* dy, int ones, long room) {
   DwSplit d;
-  if (g.O % 4 || g.M < kSplitPixels || !aligned16(dy) || gemm_force_set()) return d;
+  if (g.fp32_order || g.O % 4 || g.M < kSplitPixels || !aligned16(dy) || gemm_force_set()) return d;
   const int kp = g.C * g.KH * g.KW;
   d.tile = SplitTile{1, g.O > 32 ? 4 : 2};
   const long tiles = long(ceil_div(kp, 64)) * ceil_div(g.O, 16 * d.tile.fn);
@@ -225,7 +225,7 @@ inline bool conv_dw_split(ttrl_ctx* ctx, const ConvDwProblem<MODE>& p, const Con
 
 // Whether the split core runs the input gradient of the classes of `p`.
 inline SplitTile dx_split(const ConvGeo& g, const ConvDxProblem& p) {
-  if (g.O % 32 || g.C % 4 || gemm_force_set() || !aligned16(p.la.dy) || !aligned16(p.lb.wt) || !aligned16(p.ep.dx) ||
+  if (g.fp32_order || g.O % 32 || g.C % 4 || gemm_force_set() || !aligned16(p.la.dy) || !aligned16(p.lb.wt) || !aligned16(p.ep.dx) ||
       !aligned16(p.ep.xmask))
     return SplitTile{};
   return split_tile(p.q.M, p.q.N, p.q.groups);

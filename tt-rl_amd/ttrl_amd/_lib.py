@@ -21,6 +21,7 @@ TTRL_ESTATE = -4
 
 LAYOUT_NHWC_F32 = 0
 LAYOUT_NCHW_U8 = 1
+CONV_FP32_ORDER = 16  # or-ed into the layout of a ConvGeom
 
 # unary / binary / reduce op codes (enum order in ttrl_hip.h)
 U_OPS = ["relu", "abs", "sign", "square", "exp", "log", "tanh", "sigmoid", "sqrt", "neg",

@@ -125,6 +125,8 @@ class Conv2d(Module):
         # that writes the weight gradient fresh leaves its split-K sum to the
         # optimizer step (engine.pending).
         self.defer_bank = None
+        # Gradients summed by the FP32 matrix core alone (TTRL_CONV_FP32_ORDER).
+        self.fp32_order = False
         if weight is None:
             bound = 1.0 / math.sqrt(in_channels * kernel * kernel)
             weight = np.random.uniform(-bound, bound, (out_channels, in_channels, kernel, kernel)).astype(np.float32)
@@ -160,7 +162,7 @@ class Conv2d(Module):
     def _c_geom(self, batch: int) -> _lib.ConvGeom:
         g = self.geom
         return _lib.ConvGeom(batch, g.in_channels, g.in_h, g.in_w, g.out_channels, g.kernel, g.stride,
-                             g.padding, LAYOUTS[self.input_layout])
+                             g.padding, LAYOUTS[self.input_layout] | (_lib.CONV_FP32_ORDER if self.fp32_order else 0))
 
     # -- parameters --------------------------------------------------------
 
