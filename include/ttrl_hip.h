@@ -801,6 +801,9 @@ int ttrl_gru_step_backward(ttrl_ctx* ctx, int B, int H, const float* gi, const f
  * 16 (<= 8192); hin and W_hh 16-byte aligned. */
 int ttrl_gru_step_fused(ttrl_ctx* ctx, int B, int H, const float* gi, const float* hin, const float* W_hh,
                         const float* b_hh, float* gh, float* hout, const float* done_next, float* hin_next);
+/* ttrl_gru_step_fused for any H up to 8192 and any float alignment. */
+int ttrl_gru_step_ragged(ttrl_ctx* ctx, int B, int H, const float* gi, const float* hin, const float* W_hh,
+                         const float* b_hh, float* gh, float* hout, const float* done_next, float* hin_next);
 /* One step of the GRU's reverse walk in one launch (the backward of
  * ttrl/engine/recurrent.py:88-168 through step t): d hin_t = dhz + dgh
  * W_hh^T, where dhz = z_t * dh_t is the direct part ttrl_gru_step_backward
@@ -815,6 +818,11 @@ int ttrl_gru_step_backward_fused(ttrl_ctx* ctx, int B, int H, const float* dgh, 
                                  float* dhin, const float* gi_prev, const float* gh_prev, const float* hin_prev,
                                  const float* dout_prev, const float* done, float* dgi_prev, float* dgh_prev,
                                  float* dhz_prev);
+/* ttrl_gru_step_backward_fused for any H up to 8192 and any float alignment. */
+int ttrl_gru_step_backward_ragged(ttrl_ctx* ctx, int B, int H, const float* dgh, const float* W_hh, const float* dhz,
+                                  float* dhin, const float* gi_prev, const float* gh_prev, const float* hin_prev,
+                                  const float* dout_prev, const float* done, float* dgi_prev, float* dgh_prev,
+                                  float* dhz_prev);
 
 /* ---- GPU-resident replay -------------------------------------------------- */
 

@@ -183,3 +183,54 @@ def test_fused_steps_refuse_what_they_cannot_run(device):
     with pytest.raises(ValueError, match="given together"):
         device.call("ttrl_gru_step_backward_fused", 4, 16, x.vp, x.vp, x.vp, x.vp, x.vp, None, None, None, None,
                     None, None, None)
+
+
+@pytest.mark.parametrize("B,H", [(1, 1), (5, 7), (8, 24), (22, 250), (3, 100), (9, 33), (17, 515)])
+def test_ragged_steps_match_float64(device, B, H):
+    """The one-launch steps at hidden sizes off the 16s (tails of the units,
+    of both reductions and of the batch), operands off float4 alignment, and a
+    NaN in one sequence that must not reach the others through the reads past
+    a row's end.  Sums of up to 3H terms: rel (3H + 16) * 2^-24 of the
+    largest, taken as 1e-5 like the fused steps."""
+    from ttrl_amd.engine.tensor import DeviceArray
+
+    G = 3 * H
+    rng = np.random.default_rng(B * 1000 + H)
+    gi, hin = rng.standard_normal((B, G)), rng.standard_normal((B, H))
+    W, b = rng.standard_normal((H, G)) / np.sqrt(H), rng.standard_normal((1, G))
+    dgh, dhz, dout = rng.standard_normal((B, G)), rng.standard_normal((B, H)), rng.standard_normal((B, H))
+    done = (rng.random(B) < 0.3).astype(np.float32)
+    bad = B // 2 if B > 2 else None
+    if bad is not None:
+        hin[bad, 0] = dgh[bad, 0] = np.nan
+    ok = np.arange(B) != (-1 if bad is None else bad)
+    gi, hin, W, b, dgh, dhz, dout = (np.asarray(a, np.float32) for a in (gi, hin, W, b, dgh, dhz, dout))
+
+    def off(a):  # one float past an allocation's start
+        d = _arr(device, np.concatenate([[0.0], a.ravel()]))
+        return d, d.view(1, a.shape)
+
+    keep, (dgi_, dhin_, dW_, ddgh) = zip(*[off(a) for a in (gi, hin, W, dgh)])
+    db_, ddone, d_dhz, d_dout = (_arr(device, a) for a in (b, done, dhz, dout))
+    gh, hout, hnext = DeviceArray(device, (B, G)), DeviceArray(device, (B, H)), DeviceArray(device, (B, H))
+    device.call("ttrl_gru_step_ragged", B, H, dgi_.vp, dhin_.vp, dW_.vp, db_.vp, gh.vp, hout.vp, ddone.vp, hnext.vp)
+    gi, hin, W, dgh, dhz, dout = (a.astype(np.float64) for a in (gi, hin, W, dgh, dhz, dout))
+    gh64 = hin @ W + b[0]
+    r, z = _sig(gi[:, :H] + gh64[:, :H]), _sig(gi[:, H:2 * H] + gh64[:, H:2 * H])
+    hn = gh64[:, 2 * H:]
+    n = np.tanh(gi[:, 2 * H:] + r * hn)
+    out64 = (1 - z) * n + z * hin
+    for got, want in ((gh, gh64), (hout, out64), (hnext, out64 * (1 - done)[:, None])):
+        assert _rel(got.numpy()[ok], want[ok]) < 1e-5
+    dhin64 = dhz + dgh @ W.T
+    dh = dout + (1 - done)[:, None] * dhin64
+    dcp = dh * (1 - z) * (1 - n * n)
+    drp, dzp = dcp * hn * r * (1 - r), dh * (hin - n) * z * (1 - z)
+    d_ghp = _arr(device, gh64.astype(np.float32))
+    dhin, dhz_o = DeviceArray(device, (B, H)), DeviceArray(device, (B, H))
+    dgi_o, dgh_o = DeviceArray(device, (B, G)), DeviceArray(device, (B, G))
+    device.call("ttrl_gru_step_backward_ragged", B, H, ddgh.vp, dW_.vp, d_dhz.vp, dhin.vp, dgi_.vp, d_ghp.vp, dhin_.vp,
+                d_dout.vp, ddone.vp, dgi_o.vp, dgh_o.vp, dhz_o.vp)
+    for got, want in ((dhin, dhin64), (dgi_o, np.concatenate([drp, dzp, dcp], 1)),
+                      (dgh_o, np.concatenate([drp, dzp, dcp * r], 1)), (dhz_o, dh * z)):
+        assert _rel(got.numpy()[ok], want[ok]) < 1e-5

@@ -31,6 +31,13 @@
 // operand that runs along k in memory as one float4.  The partial tiles are
 // summed in wavefront order through LDS, so every output has one fixed
 // summation order.
+//
+// RAGGED takes any H (ttrl_gru_step_ragged): the last workgroup's units past
+// H store nothing, an operand's elements past the reduction are zeroed, and
+// rows are read as float4s at whatever 4-byte alignment they have (buffer
+// loads need no more).  Against a GEMM and a cell kernel per
+// step, forward and backward of 16 steps of 24 sequences: H 250 449 -> 216 us,
+// H 100 281 -> 169; bound by one launch and one memory round trip a step.
 #include "common.hpp"
 #include "tile_gemm.hpp"
 
@@ -158,6 +165,12 @@ __device__ __forceinline__ DiagLane diag_lane(int lane) {
   return DiagLane{c & 7, c >> 3, g, uint32_t(16 * (c >> 3) + 4 * g)};
 }
 
+// Zeroes the elements of a float4 at k .. k + 3 that lie past the reduction.
+__device__ __forceinline__ void keep_k(f32x4& v, uint32_t k, int n) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] = k + j < uint32_t(n) ? v[j] : 0.f;
+}
+
 // The pair groups [lo, hi) of this wavefront: a contiguous run, so it reads
 // whole cache lines of each operand row.
 __device__ __forceinline__ void wave_range(int wave, int np, int& lo, int& hi) {
@@ -178,6 +191,7 @@ struct GruFwdArgs {
   float* hin_next;         // [B][H] or null: h_t * (1 - done_next)
 };
 
+template <bool RAGGED>
 __global__ __launch_bounds__(kFt) void k_gru_fwd_fused(GruFwdArgs a) {
   __shared__ float part[kFw * 3 * 256];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -191,9 +205,10 @@ __global__ __launch_bounds__(kFt) void k_gru_fwd_fused(GruFwdArgs a) {
   const bool ep = tid < 64;  // wavefront 0
   const int er = r0 + t / kTile, eu = u0 + t % kTile, erc = min(er, B - 1);
   const float* gib = a.gi + long(erc) * G;
-  const float xr = gib[eu], xz = gib[H + eu], xn = gib[2 * H + eu];
-  const float br = a.bias[eu], bz = a.bias[H + eu], bn = a.bias[2 * H + eu];
-  const float h = a.hin[long(erc) * H + eu];
+  const int euc = RAGGED ? min(eu, H - 1) : eu;
+  const float xr = gib[euc], xz = gib[H + euc], xn = gib[2 * H + euc];
+  const float br = a.bias[euc], bz = a.bias[H + euc], bn = a.bias[2 * H + euc];
+  const float h = a.hin[long(erc) * H + euc];
   const float dv = *(a.done_next ? a.done_next + erc : a.bias);
   const float keep = a.done_next ? 1.f - dv : 1.f;
   // A: hin[r0 + cc][k] (one float4), B: W[k][e H + u0 + cc], k = 32p + kh + j.
@@ -215,7 +230,7 @@ __global__ __launch_bounds__(kFt) void k_gru_fwd_fused(GruFwdArgs a) {
       // 16: re-reads the last 16 k): loaded, then zeroed below
       const uint32_t k = 32u * uint32_t(min(p0 + s, hi - 1)) + L.kh;
       in[s] = p0 + s < hi && k < uint32_t(H);
-      const uint32_t kc = min(k, uint32_t(H - 16) + 4u * L.g);
+      const uint32_t kc = RAGGED ? k : min(k, uint32_t(H - 16) + 4u * L.g);
       av[s] = ldb4(rA, va + kc * 4u, 0);
 #pragma unroll
       for (int e = 0; e < 3; ++e) {
@@ -226,7 +241,8 @@ __global__ __launch_bounds__(kFt) void k_gru_fwd_fused(GruFwdArgs a) {
     __builtin_amdgcn_sched_barrier(0);  // every load of the chunk issues before the first product
 #pragma unroll
     for (int s = 0; s < kFwdChunk; ++s) {
-      const f32x4 x = in[s] ? av[s] : f32x4{0.f, 0.f, 0.f, 0.f};
+      f32x4 x = in[s] ? av[s] : f32x4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (RAGGED) keep_k(x, 32u * uint32_t(min(p0 + s, hi - 1)) + L.kh, H);
 #pragma unroll
       for (int e = 0; e < 3; ++e) acc[e] = mfma4(x, bv[s][e], acc[e]);
     }
@@ -251,7 +267,7 @@ __global__ __launch_bounds__(kFt) void k_gru_fwd_fused(GruFwdArgs a) {
     s3[e] = v;
   }
   const float hr = s3[0] + br, hz = s3[1] + bz, hn = s3[2] + bn;
-  if (er >= B) return;
+  if (er >= B || (RAGGED && eu >= H)) return;
   const float out = cell_forward(xr, xz, xn, hr, hz, hn, h);
   float* ghb = a.gh + long(er) * G;
   ghb[eu] = hr;
@@ -275,6 +291,7 @@ struct GruBwdArgs {
   float* dhz_prev;             // [B][H]  out: z_{t-1} * dh_{t-1}
 };
 
+template <bool RAGGED>
 __global__ __launch_bounds__(kFt) void k_gru_bwd_fused(GruBwdArgs a) {
   __shared__ float part[kFw * 256];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -287,12 +304,13 @@ __global__ __launch_bounds__(kFt) void k_gru_bwd_fused(GruBwdArgs a) {
   const bool cell = a.gi != nullptr;
   // Unconditional loads (see k_gru_fwd_fused); an absent operand reads a
   // buffer of the same shape and is not used.
-  const long eh = long(erc) * H + eu;
+  const int euc = RAGGED ? min(eu, H - 1) : eu;
+  const long eh = long(erc) * H + euc;
   const float dz0 = a.dhz[eh];
   const float* gib = (cell ? a.gi : a.dgh) + long(erc) * G;
   const float* ghb = (cell ? a.gh : a.dgh) + long(erc) * G;
-  const float xr = gib[eu], xz = gib[H + eu], xn = gib[2 * H + eu];
-  const float hr = ghb[eu], hz = ghb[H + eu], hn = ghb[2 * H + eu];
+  const float xr = gib[euc], xz = gib[H + euc], xn = gib[2 * H + euc];
+  const float hr = ghb[euc], hz = ghb[H + euc], hn = ghb[2 * H + euc];
   const float h = (cell ? a.hin : a.dhz)[eh];
   const float ov = (a.dout ? a.dout : a.dhz)[eh];
   const float dv = *(a.done ? a.done + erc : a.dhz);
@@ -303,7 +321,7 @@ __global__ __launch_bounds__(kFt) void k_gru_bwd_fused(GruBwdArgs a) {
   const __amdgpu_buffer_rsrc_t rA = make_res(a.dgh, uint32_t(B) * uint32_t(G) * 4u);
   const __amdgpu_buffer_rsrc_t rB = make_res(a.W, uint32_t(H) * uint32_t(G) * 4u);
   const uint32_t va = uint32_t(min(r0 + L.cc, B - 1)) * uint32_t(G) * 4u;
-  const uint32_t vb = uint32_t(u0 + L.cc) * uint32_t(G) * 4u;
+  const uint32_t vb = uint32_t(RAGGED ? min(u0 + L.cc, H - 1) : u0 + L.cc) * uint32_t(G) * 4u;
   const int np = (G + 31) >> 5;
   int lo, hi;
   wave_range(wave, np, lo, hi);
@@ -315,13 +333,21 @@ __global__ __launch_bounds__(kFt) void k_gru_bwd_fused(GruBwdArgs a) {
     for (int s = 0; s < kBwdChunk; ++s) {
       const uint32_t k = 32u * uint32_t(min(p0 + s, hi - 1)) + L.kh;
       in[s] = p0 + s < hi && k < uint32_t(G);
-      const uint32_t kc = min(k, uint32_t(G - 16) + 4u * L.g);
+      const uint32_t kc = RAGGED ? k : min(k, uint32_t(G - 16) + 4u * L.g);
       av[s] = ldb4(rA, va + kc * 4u, 0);
       bv[s] = ldb4(rB, vb + kc * 4u, 0);
     }
     __builtin_amdgcn_sched_barrier(0);  // every load of the chunk issues before the first product
 #pragma unroll
-    for (int s = 0; s < kBwdChunk; ++s) acc = mfma4(in[s] ? av[s] : f32x4{0.f, 0.f, 0.f, 0.f}, bv[s], acc);
+    for (int s = 0; s < kBwdChunk; ++s) {
+      f32x4 x = in[s] ? av[s] : f32x4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (RAGGED) {
+        const uint32_t k = 32u * uint32_t(min(p0 + s, hi - 1)) + L.kh;
+        keep_k(x, k, G);
+        keep_k(bv[s], k, G);
+      }
+      acc = mfma4(x, bv[s], acc);
+    }
   }
   const int c = lane & 15, g = lane >> 4;
 #pragma unroll
@@ -333,7 +359,7 @@ __global__ __launch_bounds__(kFt) void k_gru_bwd_fused(GruBwdArgs a) {
 #pragma unroll
   for (int w = 1; w < kFw; ++w) v += part[w * 256 + o0] + part[w * 256 + o1];
   const float dhin = v + dz0;
-  if (er >= B) return;
+  if (er >= B || (RAGGED && eu >= H)) return;
   if (a.dhin) a.dhin[long(er) * H + eu] = dhin;
   if (!cell) return;
   const float dh = dout + keep * dhin;
@@ -352,6 +378,32 @@ __global__ __launch_bounds__(kFt) void k_gru_bwd_fused(GruBwdArgs a) {
 unsigned grid_for(long n) {
   long g = (n + kGruThreads - 1) / kGruThreads;
   return unsigned(g < 1 ? 1 : (g > 4096 ? 4096 : g));
+}
+
+template <bool RAGGED>
+int gru_forward(ttrl_ctx* ctx, const GruFwdArgs& a, const char* name) {
+  if (a.B == 0) return TTRL_OK;
+  hipLaunchKernelGGL((k_gru_fwd_fused<RAGGED>), dim3(ceil_div(a.H, kTile), ceil_div(a.B, kTile)), dim3(kFt), 0,
+                     stream_of(ctx), a);
+  return check_launch(name);
+}
+
+template <bool RAGGED>
+int gru_backward(ttrl_ctx* ctx, const GruBwdArgs& a, const char* name) {
+  const bool cell = a.gi != nullptr;
+  TTRL_REQUIRE(cell ? (a.gh && a.hin && a.dgi && a.dgh_prev && a.dhz_prev)
+                    : !(a.gh || a.hin || a.dout || a.done || a.dgi || a.dgh_prev || a.dhz_prev),
+               "%s: the previous step's gi, gh, hin, dgi, dgh and dhz are given together", name);
+  TTRL_REQUIRE(cell || a.dhin, "%s: nothing to write (dhin and gi_prev both NULL)", name);
+  if (a.B == 0) return TTRL_OK;
+  hipLaunchKernelGGL((k_gru_bwd_fused<RAGGED>), dim3(ceil_div(a.H, kTile), ceil_div(a.B, kTile)), dim3(kFt), 0,
+                     stream_of(ctx), a);
+  return check_launch(name);
+}
+
+// Past its end an operand is addressed up to 64 rows or 64 k further on.
+bool gru_ragged_ok(int B, int H) {
+  return B >= 0 && H > 0 && H <= 8192 && long(B) * 3 * H * 4 < kMaxOperandBytes;
 }
 
 }  // namespace
@@ -398,10 +450,17 @@ int ttrl_gru_step_fused(ttrl_ctx* ctx, int B, int H, const float* gi, const floa
                "ttrl_gru_step_fused: H must be a positive multiple of 16 up to 8192 (got B=%d, H=%d)", B, H);
   TTRL_REQUIRE((reinterpret_cast<uintptr_t>(hin) | reinterpret_cast<uintptr_t>(W_hh)) % 16 == 0,
                "ttrl_gru_step_fused: hin and W_hh must be 16-byte aligned");
-  if (B == 0) return TTRL_OK;
-  GruFwdArgs a{B, H, gi, hin, W_hh, b_hh, gh, hout, done_next, hin_next};
-  hipLaunchKernelGGL(k_gru_fwd_fused, dim3(unsigned(H / kTile), ceil_div(B, kTile)), dim3(kFt), 0, stream_of(ctx), a);
-  return check_launch("ttrl_gru_step_fused");
+  return gru_forward<false>(ctx, GruFwdArgs{B, H, gi, hin, W_hh, b_hh, gh, hout, done_next, hin_next},
+                            "ttrl_gru_step_fused");
+}
+
+int ttrl_gru_step_ragged(ttrl_ctx* ctx, int B, int H, const float* gi, const float* hin, const float* W_hh,
+                         const float* b_hh, float* gh, float* hout, const float* done_next, float* hin_next) {
+  TTRL_REQUIRE(ctx && gi && hin && W_hh && b_hh && gh && hout, "ttrl_gru_step_ragged: null argument");
+  TTRL_REQUIRE(gru_ragged_ok(B, H), "ttrl_gru_step_ragged: H up to 8192 and operands under 2^30 bytes (got B=%d, H=%d)",
+               B, H);
+  return gru_forward<true>(ctx, GruFwdArgs{B, H, gi, hin, W_hh, b_hh, gh, hout, done_next, hin_next},
+                           "ttrl_gru_step_ragged");
 }
 
 int ttrl_gru_step_backward_fused(ttrl_ctx* ctx, int B, int H, const float* dgh, const float* W_hh, const float* dhz,
@@ -414,15 +473,19 @@ int ttrl_gru_step_backward_fused(ttrl_ctx* ctx, int B, int H, const float* dgh, 
                H);
   TTRL_REQUIRE((reinterpret_cast<uintptr_t>(dgh) | reinterpret_cast<uintptr_t>(W_hh)) % 16 == 0,
                "ttrl_gru_step_backward_fused: dgh and W_hh must be 16-byte aligned");
-  const bool cell = gi_prev != nullptr;
-  TTRL_REQUIRE(cell ? (gh_prev && hin_prev && dgi_prev && dgh_prev && dhz_prev)
-                    : !(gh_prev || hin_prev || dout_prev || done || dgi_prev || dgh_prev || dhz_prev),
-               "ttrl_gru_step_backward_fused: the previous step's gi, gh, hin, dgi, dgh and dhz are given together");
-  TTRL_REQUIRE(cell || dhin, "ttrl_gru_step_backward_fused: nothing to write (dhin and gi_prev both NULL)");
-  if (B == 0) return TTRL_OK;
-  GruBwdArgs a{B, H, dgh, W_hh, dhz, dhin, gi_prev, gh_prev, hin_prev, dout_prev, done, dgi_prev, dgh_prev, dhz_prev};
-  hipLaunchKernelGGL(k_gru_bwd_fused, dim3(unsigned(H / kTile), ceil_div(B, kTile)), dim3(kFt), 0, stream_of(ctx), a);
-  return check_launch("ttrl_gru_step_backward_fused");
+  return gru_backward<false>(ctx, GruBwdArgs{B, H, dgh, W_hh, dhz, dhin, gi_prev, gh_prev, hin_prev, dout_prev, done,
+                                             dgi_prev, dgh_prev, dhz_prev}, "ttrl_gru_step_backward_fused");
+}
+
+int ttrl_gru_step_backward_ragged(ttrl_ctx* ctx, int B, int H, const float* dgh, const float* W_hh, const float* dhz,
+                                  float* dhin, const float* gi_prev, const float* gh_prev, const float* hin_prev,
+                                  const float* dout_prev, const float* done, float* dgi_prev, float* dgh_prev,
+                                  float* dhz_prev) {
+  TTRL_REQUIRE(ctx && dgh && W_hh && dhz, "ttrl_gru_step_backward_ragged: null argument");
+  TTRL_REQUIRE(gru_ragged_ok(B, H),
+               "ttrl_gru_step_backward_ragged: H up to 8192 and operands under 2^30 bytes (got B=%d, H=%d)", B, H);
+  return gru_backward<true>(ctx, GruBwdArgs{B, H, dgh, W_hh, dhz, dhin, gi_prev, gh_prev, hin_prev, dout_prev, done,
+                                            dgi_prev, dgh_prev, dhz_prev}, "ttrl_gru_step_backward_ragged");
 }
 
 }  // extern "C"

@@ -344,6 +344,7 @@ class PPOLearner:
         # gradient bank of the device context; the step forms them all in one
         # launch when it settles the gradients before the clip.
         from ttrl_amd.engine.conv import Conv2d
+        from ttrl_amd.engine.recurrent import GRUCell
         from ttrl_amd.nets.acting import _walk_modules
 
         convs = [m for _, m in _walk_modules(self.net) if isinstance(m, Conv2d)]
@@ -357,6 +358,8 @@ class PPOLearner:
         # against 4.86 (minibatches of 256, 16 steps).
         for conv in convs:
             conv.fp32_order = True
+        for m in (m for _, m in _walk_modules(self.net) if isinstance(m, GRUCell)):
+            m.two_launch_steps = True  # the same, at hidden sizes off the 16s
         self._rng = np.random.default_rng(seed)
         self.frame_count = 0
         self.update_count = 0

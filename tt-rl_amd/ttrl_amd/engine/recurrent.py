@@ -32,6 +32,11 @@ from ttrl_amd.engine.tensor import DeviceArray
 __all__ = ["GATES", "GRU", "GRUCell"]
 
 GATES = ("reset", "update", "candidate")
+# Workgroups (8 units x 8 sequences each) up to which a ragged step runs in one
+# launch: past two to three a CU the GEMM's larger tiles read less.  Forward
+# and backward of 8 steps: H 515, 64 sequences (520) 307 -> 279 us, 128 (1040)
+# 374 -> 420; H 250, 128 sequences (512) 264 -> 186.
+_RAGGED_GROUPS = 640
 
 
 class GRUCell(Module):
@@ -43,6 +48,9 @@ class GRUCell(Module):
                              f"hidden_size={hidden_size}")
         self.in_features = int(in_features)
         self.hidden_size = int(hidden_size)
+        # A hidden size off the 16s keeps a GEMM and a cell kernel per step,
+        # whose sums have another order (RecurrentPPOLearner).
+        self.two_launch_steps = False
         gates = len(GATES) * self.hidden_size
         bound = 1.0 / math.sqrt(self.hidden_size)
 
@@ -131,9 +139,11 @@ def unroll(cell: GRUCell, x: Tensor, h0: Tensor, done: Tensor | None):
         return arr.view(t * B * width, (B, width))
 
     W_hh = cell.weight_hh.data
-    # One launch per step when the fused kernels' layout holds (H a multiple
-    # of 16, float4-aligned operands), else a GEMM and a cell kernel per step.
-    fused = H % 16 == 0 and H <= 8192 and all(a.ptr % 16 == 0 for a in (HIN, W_hh))
+    # One launch per step, else a GEMM and a cell kernel per step.  Off the
+    # fused kernels' own layout (H a multiple of 16, float4-aligned operands)
+    # the ragged form while its workgroups are few.
+    step = "fused" if H % 16 == 0 and all(a.ptr % 16 == 0 for a in (HIN, W_hh)) else "ragged"
+    fused = H <= 8192 and (step == "fused" or (-(-H // 8) * -(-B // 8) <= _RAGGED_GROUPS and not cell.two_launch_steps))
     _linear(dev, X, cell.weight_ih, cell.bias_ih, GI, T * B, F, G)
     dev.call("ttrl_gru_mask", B, H, h0.data.vp, done_at(0), HIN.vp)
     for t in range(T):
@@ -142,7 +152,7 @@ def unroll(cell: GRUCell, x: Tensor, h0: Tensor, done: Tensor | None):
         done_next = None if last else done_at(t + 1)
         hin_next = None if last else at(HIN, t + 1, H).vp
         if fused:
-            dev.call("ttrl_gru_step_fused", B, H, gi.vp, hin.vp, W_hh.vp, cell.bias_hh.data.vp, gh.vp, out.vp,
+            dev.call("ttrl_gru_step_" + step, B, H, gi.vp, hin.vp, W_hh.vp, cell.bias_hh.data.vp, gh.vp, out.vp,
                      done_next, hin_next)
         else:
             _linear(dev, hin, cell.weight_hh, cell.bias_hh, gh, B, H, G)
@@ -161,13 +171,13 @@ def unroll(cell: GRUCell, x: Tensor, h0: Tensor, done: Tensor | None):
         dev.call("ttrl_gru_step_backward", B, H, at(GI, last, G).vp, at(GH, last, G).vp, at(HIN, last, H).vp,
                  at(grad, last, H).vp, None, None, at(DGI, last, G).vp, at(DGH, last, G).vp, DHZ[last % 2].vp)
         for s in range(last, 0, -1):
-            dev.call("ttrl_gru_step_backward_fused", B, H, at(DGH, s, G).vp, W_hh.vp, DHZ[s % 2].vp, None,
+            dev.call("ttrl_gru_step_backward_" + step, B, H, at(DGH, s, G).vp, W_hh.vp, DHZ[s % 2].vp, None,
                      at(GI, s - 1, G).vp, at(GH, s - 1, G).vp, at(HIN, s - 1, H).vp, at(grad, s - 1, H).vp,
                      done_at(s), at(DGI, s - 1, G).vp, at(DGH, s - 1, G).vp, DHZ[(s - 1) % 2].vp)
         if not need_h0:
             return None
         dhin0 = DeviceArray(dev, (B, H))
-        dev.call("ttrl_gru_step_backward_fused", B, H, at(DGH, 0, G).vp, W_hh.vp, DHZ[0].vp, dhin0.vp,
+        dev.call("ttrl_gru_step_backward_" + step, B, H, at(DGH, 0, G).vp, W_hh.vp, DHZ[0].vp, dhin0.vp,
                  None, None, None, None, None, None, None, None)
         return dhin0
 
