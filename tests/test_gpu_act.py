@@ -382,3 +382,25 @@ def test_direct_replay_gives_the_graph_launch_bits(device):
             trace.set_direct(True)
     finally:
         trace.close()
+
+
+@pytest.mark.parametrize("B,K,A", [(1, 1, 1), (3, 255, 8), (4, 256, 9), (5, 257, 16), (6, 300, 17), (2, 513, 32)])
+def test_q_act_weights_staged_in_rounds(device, B, K, A):
+    """Reduction lengths around a round of staged weight rows, widths around
+    each instantiation's, batches that end inside a workgroup.  K products of
+    which each lane adds K / 64 and the butterfly six sums: (K / 64 + 8)
+    roundings of at most 2^-24 of the sum of magnitudes."""
+    rng = np.random.default_rng(K)
+    h, W = rng.standard_normal((B, K)).astype(np.float32), rng.standard_normal((K, A)).astype(np.float32)
+    from ttrl_amd.engine.tensor import DeviceArray
+
+    dh, dW, q = DeviceArray(device, (B, K)), DeviceArray(device, (K, A)), DeviceArray(device, (B, A))
+    act = DeviceArray(device, (B,), np.int32)
+    dh.upload(h)
+    dW.upload(W)
+    device.call("ttrl_q_act", B, K, A, dh.ptr, dW.ptr, None, q.ptr, act.ptr)
+    want = h.astype(np.float64) @ W.astype(np.float64)
+    bound = (K / 64 + 8) * 2.0 ** -24 * (np.abs(h).astype(np.float64) @ np.abs(W).astype(np.float64))
+    got = q.numpy()
+    assert np.all(np.abs(got - want) <= bound)
+    assert np.array_equal(act.numpy(), np.argmax(got, 1))

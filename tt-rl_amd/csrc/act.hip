@@ -18,6 +18,11 @@
 // each column are combined by an xor butterfly, which leaves the identical
 // total in every lane, so any lane can take the decision.  The layer is tiny
 // (K <= a few thousand, N <= 32): latency, not bandwidth or MFMA, bounds it.
+// Wide heads (N > 8) of more than one row take the weights through LDS: a
+// lane reading its own weight rows touches a cache line per lane and element
+// (K 300, N 16: 4 rows 13.4 us, 1,000 rows 14.2; staged 9.9 and 10.8).  One
+// row alone waits longer for the staging than for its own reads (9.0 / 10.1),
+// and so does a narrow head at any batch (K 512, N 6: 5.2 to 6.1 / 6.5 to 7.7).
 #include "common.hpp"
 
 #include <cmath>
@@ -28,7 +33,8 @@ namespace {
 constexpr int kActThreads = 256;  // four wavefronts, four lane rows per workgroup
 constexpr int kActRows = kActThreads / 64;
 constexpr int kActMaxN = 32;
-constexpr int kActDepth = 4;  // columns per lane whose loads are in flight together
+constexpr int kActDepth = 4;               // columns per lane of one round
+constexpr int kActCols = 64 * kActDepth;   // weight rows staged per round
 constexpr float kActLog2 = 0.69314718055994530942f;
 constexpr float kActLog2Pi = 1.83787706640934548356f;
 
@@ -53,6 +59,7 @@ struct ActArgs {
   float* action;  // squashed: [B][n1]
   float* logp;    // squashed: [B]
   float* u;       // squashed: [B][n1] pre-squash sample, or null
+  FDiv d1, d2;    // division by n1 and by N - n1
 };
 
 __device__ __forceinline__ float softplus_act(float x) {
@@ -60,11 +67,11 @@ __device__ __forceinline__ float softplus_act(float x) {
   return r + logf(expf(-fabsf(x)) + 1.f);
 }
 
-template <ActMode MODE, int NP>
+template <ActMode MODE, int NP, bool STAGED>
 __global__ __launch_bounds__(kActThreads) void k_head_act(ActArgs a) {
-  const int lane = threadIdx.x & 63;
-  const int b = blockIdx.x * kActRows + (threadIdx.x >> 6);
-  if (b >= a.B) return;  // uniform per wavefront
+  __shared__ float wt[STAGED ? kActCols * (NP + 1) : 1];  // odd pitch: a column's 64 lanes hit 64 banks
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int row = blockIdx.x * kActRows + (tid >> 6), b = min(row, a.B - 1);
   const int N = a.N, n1 = a.n1, n2 = a.N - a.n1;
   const float* hb = a.h + long(b) * a.K;
   float acc[NP];
@@ -82,38 +89,76 @@ __global__ __launch_bounds__(kActThreads) void k_head_act(ActArgs a) {
     if (a.b1) bias_mu = a.b1[own];
     if (a.b2) bias_ls = a.b2[own];
   }
-  // kActDepth columns per lane in flight at once: a round's loads are all
-  // issued before its products, so a row pays one memory latency per
-  // 64 * kActDepth columns; the columns past the last whole round follow
-  // one at a time.  Each lane sums its columns in ascending k.
-  int k0 = lane;
-  for (; k0 + 64 * (kActDepth - 1) < a.K; k0 += 64 * kActDepth) {
-    float x[kActDepth], w[kActDepth][NP];
+  if constexpr (STAGED) {
+    // kActCols rows of the weights at a time, read once per workgroup in memory
+    // order and laid out by row in LDS; every load of a round is issued before
+    // the first is waited for (past the round's end a thread repeats the last
+    // element and stores nothing).  Each lane sums its columns in ascending k.
+    for (int c0 = 0; c0 < a.K; c0 += kActCols) {
+      const int cols = min(kActCols, a.K - c0), c1 = cols * n1, all = cols * N;
+      const float* w1 = a.W1 + long(c0) * n1;
+      const float* w2 = a.W2 + long(c0) * n2;
+      float x[kActDepth], w[NP];
 #pragma unroll
-    for (int r = 0; r < kActDepth; ++r) {
-      const int k = k0 + 64 * r;
-      x[r] = hb[k];
+      for (int r = 0; r < kActDepth; ++r) x[r] = hb[min(c0 + lane + 64 * r, a.K - 1)];
+#pragma unroll
+      for (int j = 0; j < NP; ++j) {
+        const int i = min(tid + kActThreads * j, all - 1);
+        w[j] = *(i < c1 ? w1 + i : w2 + (i - c1));
+      }
+      if (c0) __syncthreads();
+#pragma unroll
+      for (int j = 0; j < NP; ++j) {
+        const int i = tid + kActThreads * j;
+        const bool first = i < c1;
+        const int e = first ? i : i - c1, k = first ? a.d1.div(e) : a.d2.div(e);
+        if (i < all) wt[k * (NP + 1) + (first ? e - k * n1 : n1 + e - k * n2)] = w[j];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < kActDepth; ++r)
+        if (lane + 64 * r < cols) {
+          const float* wr = wt + (lane + 64 * r) * (NP + 1);
+#pragma unroll
+          for (int n = 0; n < NP; ++n)
+            if (n < N) acc[n] += x[r] * wr[n];
+        }
+    }
+  } else {
+    // kActDepth columns per lane in flight at once: a round's loads are all
+    // issued before its products, so a row pays one memory latency per
+    // 64 * kActDepth columns; the columns past the last whole round follow
+    // one at a time.  Each lane sums its columns in ascending k.
+    int k0 = lane;
+    for (; k0 + 64 * (kActDepth - 1) < a.K; k0 += 64 * kActDepth) {
+      float x[kActDepth], w[kActDepth][NP];
+#pragma unroll
+      for (int r = 0; r < kActDepth; ++r) {
+        const int k = k0 + 64 * r;
+        x[r] = hb[k];
+        const float* w1 = a.W1 + long(k) * n1;
+        const float* w2 = a.W2 + long(k) * n2;
+#pragma unroll
+        for (int n = 0; n < NP; ++n) w[r][n] = n < n1 ? w1[n] : n < N ? w2[n - n1] : 0.f;
+      }
+#pragma unroll
+      for (int r = 0; r < kActDepth; ++r)
+#pragma unroll
+        for (int n = 0; n < NP; ++n)
+          if (n < N) acc[n] += x[r] * w[r][n];
+    }
+    for (int k = k0; k < a.K; k += 64) {
+      const float x = hb[k];
       const float* w1 = a.W1 + long(k) * n1;
       const float* w2 = a.W2 + long(k) * n2;
 #pragma unroll
-      for (int n = 0; n < NP; ++n) w[r][n] = n < n1 ? w1[n] : n < N ? w2[n - n1] : 0.f;
-    }
-#pragma unroll
-    for (int r = 0; r < kActDepth; ++r)
-#pragma unroll
-      for (int n = 0; n < NP; ++n)
-        if (n < N) acc[n] += x[r] * w[r][n];
-  }
-  for (int k = k0; k < a.K; k += 64) {
-    const float x = hb[k];
-    const float* w1 = a.W1 + long(k) * n1;
-    const float* w2 = a.W2 + long(k) * n2;
-#pragma unroll
-    for (int n = 0; n < NP; ++n) {
-      if (n < n1) acc[n] += x * w1[n];
-      else if (n < N) acc[n] += x * w2[n - n1];
+      for (int n = 0; n < NP; ++n) {
+        if (n < n1) acc[n] += x * w1[n];
+        else if (n < N) acc[n] += x * w2[n - n1];
+      }
     }
   }
+  if (row >= a.B) return;
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
 #pragma unroll
@@ -184,14 +229,16 @@ __global__ __launch_bounds__(kActThreads) void k_head_act(ActArgs a) {
 }
 
 template <ActMode MODE>
-int launch_head_act(ttrl_ctx* ctx, const ActArgs& a, int width, const char* name) {
-  const dim3 grid(unsigned((a.B + kActRows - 1) / kActRows));
-  if (width <= 8)
-    hipLaunchKernelGGL((k_head_act<MODE, 8>), grid, dim3(kActThreads), 0, stream_of(ctx), a);
-  else if (width <= 16)
-    hipLaunchKernelGGL((k_head_act<MODE, 16>), grid, dim3(kActThreads), 0, stream_of(ctx), a);
-  else
-    hipLaunchKernelGGL((k_head_act<MODE, 32>), grid, dim3(kActThreads), 0, stream_of(ctx), a);
+int launch_head_act(ttrl_ctx* ctx, ActArgs a, int width, const char* name) {
+  a.d1.set(a.n1);
+  a.d2.set(a.N > a.n1 ? a.N - a.n1 : 1);
+  const dim3 grid(unsigned((a.B + kActRows - 1) / kActRows)), block(kActThreads);
+  const bool staged = a.B > 1;
+  if (width <= 8) hipLaunchKernelGGL((k_head_act<MODE, 8, false>), grid, block, 0, stream_of(ctx), a);
+  else if (width <= 16 && staged) hipLaunchKernelGGL((k_head_act<MODE, 16, true>), grid, block, 0, stream_of(ctx), a);
+  else if (width <= 16) hipLaunchKernelGGL((k_head_act<MODE, 16, false>), grid, block, 0, stream_of(ctx), a);
+  else if (staged) hipLaunchKernelGGL((k_head_act<MODE, 32, true>), grid, block, 0, stream_of(ctx), a);
+  else hipLaunchKernelGGL((k_head_act<MODE, 32, false>), grid, block, 0, stream_of(ctx), a);
   return check_launch(name);
 }
 

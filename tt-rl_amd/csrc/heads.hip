@@ -17,6 +17,7 @@
 #include "common.hpp"
 #include "dqn_row.hpp"
 
+#include <algorithm>
 #include <cmath>
 
 namespace ttrl {
@@ -303,36 +304,39 @@ __global__ __launch_bounds__(kHeadThreads) void k_sac_sample(int B, int d, const
 }
 
 // Backward of k_sac_sample to the head's [mean | log_std] outputs.
-// g_action0 (+ g_action1): dL/d action; g_logp: dL/d logp per row.
+// g_action0 (+ g_action1): dL/d action; g_logp: dL/d logp per row.  One thread
+// per element: a thread per row walked its d elements one memory round trip
+// after another (500 rows, d 8: 11.0 us, now 4.6).
 __global__ __launch_bounds__(kHeadThreads) void k_sac_sample_bwd(
-    int B, int d, const float* __restrict__ head, const float* __restrict__ noise, const float* __restrict__ u_in,
-    const float* __restrict__ half_width, const float* __restrict__ g_action0, const float* __restrict__ g_action1,
-    const float* __restrict__ g_logp, float lo, float hi, float* __restrict__ d_head, float beta) {
-  for (int b = blockIdx.x * kHeadThreads + threadIdx.x; b < B; b += gridDim.x * kHeadThreads) {
+    int B, int d, FDiv dd, const float* __restrict__ head, const float* __restrict__ noise,
+    const float* __restrict__ u_in, const float* __restrict__ half_width, const float* __restrict__ g_action0,
+    const float* __restrict__ g_action1, const float* __restrict__ g_logp, float lo, float hi,
+    float* __restrict__ d_head, float beta) {
+  const int n = B * d;
+  for (int e = blockIdx.x * kHeadThreads + threadIdx.x; e < n; e += gridDim.x * kHeadThreads) {
+    const int b = dd.div(e), i = e - b * d;
     const float* hb = head + long(b) * 2 * d;
     const float glp = g_logp ? g_logp[b] : 0.f;
-    for (int i = 0; i < d; ++i) {
-      const float mu = hb[i], ls = hb[d + i];
-      const float sigma = expf(ls);
-      const float eps = noise[long(b) * d + i];
-      const float u = u_in[long(b) * d + i];
-      const float z = (u - mu) / sigma;
-      const float t = tanhf(u);
-      float ga = 0.f;
-      if (g_action0) ga += g_action0[long(b) * d + i];
-      if (g_action1) ga += g_action1[long(b) * d + i];
-      // d logp / d u (explicit): -z/sigma from the Gaussian, +2 tanh(u) from
-      // the squash correction; d logp / d mean (explicit) = z/sigma;
-      // d logp / d log_std (explicit) = z^2 - 1.
-      const float gu = ga * half_width[i] * (1.f - t * t) + glp * (2.f * t - z / sigma);
-      const float gmu = gu + glp * (z / sigma);
-      float gls = gu * (sigma * eps) + glp * (z * z - 1.f);
-      gls = (ls > lo && ls < hi) ? gls : 0.f;
-      float* dm = d_head + long(b) * 2 * d + i;
-      float* dl = d_head + long(b) * 2 * d + d + i;
-      *dm = beta != 0.f ? *dm * beta + gmu : gmu;
-      *dl = beta != 0.f ? *dl * beta + gls : gls;
-    }
+    const float mu = hb[i], ls = hb[d + i];
+    const float sigma = expf(ls);
+    const float eps = noise[e];
+    const float u = u_in[e];
+    const float z = (u - mu) / sigma;
+    const float t = tanhf(u);
+    float ga = 0.f;
+    if (g_action0) ga += g_action0[e];
+    if (g_action1) ga += g_action1[e];
+    // d logp / d u (explicit): -z/sigma from the Gaussian, +2 tanh(u) from
+    // the squash correction; d logp / d mean (explicit) = z/sigma;
+    // d logp / d log_std (explicit) = z^2 - 1.
+    const float gu = ga * half_width[i] * (1.f - t * t) + glp * (2.f * t - z / sigma);
+    const float gmu = gu + glp * (z / sigma);
+    float gls = gu * (sigma * eps) + glp * (z * z - 1.f);
+    gls = (ls > lo && ls < hi) ? gls : 0.f;
+    float* dm = d_head + long(b) * 2 * d + i;
+    float* dl = d_head + long(b) * 2 * d + d + i;
+    *dm = beta != 0.f ? *dm * beta + gmu : gmu;
+    *dl = beta != 0.f ? *dl * beta + gls : gls;
   }
 }
 
@@ -482,8 +486,17 @@ int ttrl_sac_sample_backward(ttrl_ctx* ctx, int B, int d, const float* head, con
                              const float* g_logp, float log_std_min, float log_std_max, float* d_head, float beta) {
   TTRL_REQUIRE(ctx && head && noise && u && half_width && d_head, "ttrl_sac_sample_backward: null argument");
   TTRL_REQUIRE(B > 0 && d > 0, "ttrl_sac_sample_backward: empty batch");
-  hipLaunchKernelGGL(k_sac_sample_bwd, dim3(rows_grid(B)), dim3(kHeadThreads), 0, stream_of(ctx), B, d, head,
-                     noise, u, half_width, g_action0, g_action1, g_logp, log_std_min, log_std_max, d_head, beta);
+  FDiv dd;
+  dd.set(d);
+  const int most = std::max(1, (1 << 30) / d);  // rows whose elements an int counts
+  for (long b0 = 0; b0 < B; b0 += most) {
+    const int rows = int(std::min<long>(most, B - b0));
+    const long o = b0 * d;
+    hipLaunchKernelGGL(k_sac_sample_bwd, dim3(std::min(rows_grid(rows * d), 65535u)), dim3(kHeadThreads), 0,
+                       stream_of(ctx), rows, d, dd, head + 2 * o, noise + o, u + o, half_width,
+                       g_action0 ? g_action0 + o : nullptr, g_action1 ? g_action1 + o : nullptr,
+                       g_logp ? g_logp + b0 : nullptr, log_std_min, log_std_max, d_head + 2 * o, beta);
+  }
   return check_launch("ttrl_sac_sample_backward");
 }
 
