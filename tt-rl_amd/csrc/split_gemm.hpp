@@ -89,84 +89,6 @@ __device__ __forceinline__ f32x4 mfma_bf16(const u32x4& a, const u32x4& b, const
 // of the step, so each load takes 64 contiguous bytes of a row from its
 // four lanes; without, k = 8 lg .. 8 lg + 7.  B is stored to match.
 
-// v(r, k) = p[g][r*ld + k]; 16-byte rows.
-struct SaRow {
-  const float* p[kMaxGroups] = {};
-  long ld = 0;
-  int rows = 0, K = 0;
-  __host__ __device__ long bytes() const { return rows > 0 ? ((long(rows) - 1) * ld + K) * 4 : 0; }
-  struct Params {
-    const float* p;
-    uint32_t bytes;
-    int ld, rows, K;
-  };
-  struct Live {
-    static constexpr bool EXACT = false, PERM = true, TABLE = false;
-    Params q;
-    __amdgpu_buffer_rsrc_t rs;
-    struct Raw { f32x4 a, b; };
-    using Row = uint32_t;
-    __device__ __forceinline__ uint32_t row(int r, int lg) const {
-      return r < q.rows ? uint32_t(r * q.ld) * 4u + uint32_t(lg) * 16u : kBad;
-    }
-    __device__ __forceinline__ uint32_t kbase(int k0) const { return k0 < q.K ? uint32_t(k0) * 4u : kBad; }
-    __device__ __forceinline__ void issue(uint32_t row, uint32_t kb, Raw& f) const {
-      f.a = ld_f4(rs, row + kb);
-      f.b = ld_f4(rs, row + kb + 64u);
-    }
-    __device__ __forceinline__ void resolve(const Raw& f, f32x4& a, f32x4& b) const {
-      a = f.a;
-      b = f.b;
-    }
-  };
-  __device__ __forceinline__ Live live(int g) const {
-    const Params q = pin_pod(Params{p[g], uint32_t(bytes()), int(ld), rows, K});
-    return Live{q, make_res(q.p, q.bytes)};
-  }
-};
-
-// v(r, k) = p[g][k*ld + r]: a transposed operand (a weight gradient's layer
-// input).  A lane's 8 k are 8 rows of memory, its 16-lane group 64 contiguous
-// bytes of each.
-struct SaColT {
-  const float* p[kMaxGroups] = {};
-  long ld = 0;
-  int rows = 0, K = 0;
-  __host__ __device__ long bytes() const { return K > 0 && rows > 0 ? ((long(K) - 1) * ld + rows) * 4 : 0; }
-  struct Params {
-    const float* p;
-    uint32_t bytes;
-    int ld, rows, K;
-  };
-  struct Live {
-    static constexpr bool EXACT = false, PERM = false, TABLE = false;
-    Params q;
-    __amdgpu_buffer_rsrc_t rs;
-    struct Raw { f32x4 a, b; };
-    using Row = uint32_t;
-    __device__ __forceinline__ uint32_t row(int r, int lg) const {
-      return r < q.rows ? uint32_t(r + lg * 8 * q.ld) * 4u : kBad;
-    }
-    __device__ __forceinline__ uint32_t kbase(int k0) const { return uint32_t(k0 * q.ld) * 4u; }
-    __device__ __forceinline__ void issue(uint32_t row, uint32_t kb, Raw& f) const {
-      const uint32_t o = row + kb, step = uint32_t(q.ld) * 4u;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        f.a[j] = ld_f1(rs, o + uint32_t(j) * step);
-        f.b[j] = ld_f1(rs, o + uint32_t(j + 4) * step);
-      }
-    }
-    __device__ __forceinline__ void resolve(const Raw& f, f32x4& a, f32x4& b) const {
-      a = f.a;
-      b = f.b;
-    }
-  };
-  __device__ __forceinline__ Live live(int g) const {
-    const Params q = pin_pod(Params{p[g], uint32_t(bytes()), int(ld), rows, K});
-    return Live{q, make_res(q.p, q.bytes)};
-  }
-};
-
 // ---------------------------------------------------------- B operands ---
 //
 // Vector loads only, no element paths: a branch in the loop that only some
@@ -198,33 +120,6 @@ struct SbCol {
     __device__ __forceinline__ uint32_t kbytes() const { return uint32_t(q.ld) * 4u; }
     __device__ __forceinline__ float elem(int n, int k) const {
       return ld_f1(rs, n < q.rows && k < q.K ? uint32_t(k * q.ld + n) * 4u : kBad);
-    }
-  };
-  __device__ __forceinline__ Live live(int g) const {
-    const Params q = pin_pod(Params{p[g], uint32_t(bytes()), int(ld), rows, K});
-    return Live{q, make_res(q.p, q.bytes)};
-  }
-};
-
-// v(n, k) = p[g][n*ld + k]; four k a load: 16-byte rows, K a multiple of 32.
-struct SbRow {
-  const float* p[kMaxGroups] = {};
-  long ld = 0;
-  int rows = 0, K = 0;
-  __host__ __device__ long bytes() const { return rows > 0 ? ((long(rows) - 1) * ld + K) * 4 : 0; }
-  struct Params {
-    const float* p;
-    uint32_t bytes;
-    int ld, rows, K;
-  };
-  struct Live {
-    static constexpr bool COL = false;
-    Params q;
-    __amdgpu_buffer_rsrc_t rs;
-    __device__ __forceinline__ uint32_t row(int n) const { return n < q.rows ? uint32_t(n * q.ld) * 4u : kBad; }
-    __device__ __forceinline__ uint32_t kbase(int k0) const { return k0 < q.K ? uint32_t(k0) * 4u : kBad; }
-    __device__ __forceinline__ float elem(int n, int k) const {
-      return ld_f1(rs, n < q.rows && k < q.K ? uint32_t(n * q.ld + k) * 4u : kBad);
     }
   };
   __device__ __forceinline__ Live live(int g) const {
