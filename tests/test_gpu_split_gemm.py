@@ -41,8 +41,8 @@ def _scatter(cols, shape, k, s):
 
 def _bound(terms, magnitude):
     """Rounding of a float32 sum of `terms` products in any order: terms + 16
-    roundings (the split's dropped parts and the epilogue among the 16) of at
-    most 2^-24 of the sum of magnitudes."""
+    roundings (the split's dropped parts, at most 2^-24 of each product, and
+    the epilogue among the 16) of at most 2^-24 of the sum of magnitudes."""
     return (terms + 16) * 2.0 ** -24 * magnitude
 
 
@@ -143,3 +143,37 @@ def test_values_outside_the_split(dev, value):
             assert np.array_equal(np.sign(got[some]), np.sign(want[some]))
             fine = ~bad & (magnitude < 1e38)
             assert np.all(np.abs(got - want)[fine] <= _bound(terms, magnitude[fine]))
+
+
+def test_short_sums_of_the_worst_operands(dev):
+    """Sums of 32 products (one step of the core) of operands whose mantissa
+    leaves most in the lower parts (0x00ffff).  In 2^-24 of the sum: 1 for the
+    products left out, 1 for each of at most four additions of the main sum, 1
+    for adding the lower products' sum."""
+    rng = np.random.default_rng(5)
+    one = np.array([0x3F80FFFF], np.uint32).view(np.float32)[0]
+    x = np.ones((512, 8, 8, 32), np.float32)
+    wt = one * np.exp2(rng.integers(-3, 4, (4 * 32, 32))).astype(np.float32)
+    dy = one * np.exp2(rng.integers(-3, 4, (512 * 16, 32))).astype(np.float32)
+    _, _, dx = _backward(dev, x, dy, wt, 2, 2, False)
+    want = _scatter(dy.astype(np.float64) @ wt.astype(np.float64).T, x.shape, 2, 2)
+    assert np.max(np.abs(dx - want) / want) <= 6 * 2.0 ** -24
+
+
+def test_sums_of_one_sign_are_not_biased(dev):
+    """Rounding to nearest errs to either side alike: over n sums of positive
+    terms, each off by at most E * 2^-24 of itself, the mean error lies within
+    five standard deviations, 5 E / sqrt(n) * 2^-24 (E = 12 bounds the largest
+    of either gradient)."""
+    rng = np.random.default_rng(6)
+    k, s = 4, 2
+    x = np.abs(rng.standard_normal((256, 20, 20, 32))).astype(np.float32)
+    wt = np.abs(rng.standard_normal((k * k * 32, 64))).astype(np.float32)
+    a = _patches(x, k, s)
+    dy = np.abs(rng.standard_normal((a.shape[0], 64))).astype(np.float32)
+    dw, _, dx = _backward(dev, x, dy, wt, k, s, False)
+    g = dy.astype(np.float64)
+    for got, want in ((dw, a.T @ g), (dx, _scatter(g @ wt.astype(np.float64).T, x.shape, k, s))):
+        e = (got - want) / want * 2.0 ** 24
+        assert np.max(np.abs(e)) <= 12
+        assert abs(e.mean()) <= 5 * 12 / np.sqrt(e.size)

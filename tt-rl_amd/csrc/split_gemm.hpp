@@ -1,20 +1,27 @@
 // FP32 products on the bf16 matrix cores of gfx950.
 //
-// A float is exactly the sum of three bf16 numbers: its upper 16 bits, the
-// upper 16 bits of what is left, and the rest (8 significant bits each).  A
-// product of two floats is then nine bf16 products, of which the six largest
-// are kept, each exact in FP32 and added in FP32 by the matrix core: what is
-// left out is under 2^-24 of the product, and 16x16x32 bf16 MFMA runs six of
-// them in 3/8 of the time 16x16x4 FP32 MFMA takes for the product.  Bytes
-// (uint8 frames) are exact in one bf16, so they take three.
+// A float is exactly the sum of three bf16 numbers: the float rounded to the
+// nearest bf16, what is left rounded likewise, and the rest (8 significant
+// bits each, either sign; Henry, Tang and Heinecke, "Leveraging the bfloat16
+// Artificial Intelligence Datatype For Higher-Precision Computations", ARITH
+// 2019).  A product of two floats is then nine bf16 products, of which the six
+// largest are kept, each exact in FP32 and added in FP32 by the matrix core.
+// The parts are at most 2^-8 and 2^-17 of the operand's power of two, so what
+// is left out is at most 2^-24 + 2^-34 of the product, of either sign, and
+// 16x16x32 bf16 MFMA runs six of them in 3/8 of the time 16x16x4 FP32 MFMA
+// takes for the product.  (Parts cut off instead of rounded leave out up to
+// 2^-21, always towards zero: a sum of positive terms came out 0.69 * 2^-24
+// low, rounded parts leave its mean error at 0.005 * 2^-24.)  Bytes (uint8
+// frames) are exact in one bf16, so they take three.
 //
 // What it gives (both gradients of a Nature-CNN layer, batch 256; FP32 core
-// before): second layer 58.1 -> 41.9 us, third 46.4 -> 36.6; batch 1024 222 ->
-// 124 and 154 -> 89.  The error against float64 falls, since the main sum is
-// rounded once per 32 k: weight gradients at batch 1024 6.8e-7 -> 2.3e-7, input
-// gradients 2.7e-7 -> 1.0e-7.  What bounds it: a stage's chain of loads, splits
-// (5.5 VALU instructions per float) and LDS round trips; the matrix core is
-// busy about a third of the time.
+// before): second layer 62.2 -> 45.4 us, third 50.5 -> 39.4; batch 1024 and 512
+// 196.5 -> 118.4 and 88.1 -> 55.1.  The error against float64 falls, since the
+// main sum is rounded once per 32 k: weight gradients at batch 1024 6.9e-7 ->
+// 2.2e-7, input gradients 2.7e-7 -> 8.5e-8, at K = 32 (2 x 2 kernels, stride 2)
+// 1.0e-7 -> 3.9e-8.  What bounds it: a stage's chain of loads, splits (5.5 VALU
+// instructions per float) and LDS round trips; the matrix core is busy about a
+// third of the time.
 //
 // One workgroup owns BM x BN of the output, NW wavefronts along M, each
 // WM x FN fragments of 16 x 16.
@@ -40,19 +47,26 @@ namespace ttrl {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ uint32_t hi_pair(float a, float b) {  // upper halves of (a, b), a in the low half
   return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
 }
-__device__ __forceinline__ float low_part(float x) { return x - __uint_as_float(__float_as_uint(x) & 0xffff0000u); }
+// (a, b) to the nearest bf16 pair, left as a's and b's rest (exact).
+__device__ __forceinline__ uint32_t take_nearest(float& a, float& b) {
+  uint32_t p = __builtin_bit_cast(uint32_t, bf16x2{__bf16(a), __bf16(b)});  // v_cvt_pk_bf16_f32
+  asm("" : "+v"(p));  // else the lower half is converted again on its own
+  a -= __uint_as_float(p << 16);
+  b -= __uint_as_float(p & 0xffff0000u);
+  return p;
+}
 
 // The three planes of a pair of floats.
 __device__ __forceinline__ void split2(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
-  h = hi_pair(a, b);
-  const float a1 = low_part(a), b1 = low_part(b);
-  m = hi_pair(a1, b1);
-  l = hi_pair(low_part(a1), low_part(b1));
+  h = take_nearest(a, b);
+  m = take_nearest(a, b);
+  l = hi_pair(a, b);  // at most 8 significant bits are left
 }
 
 struct Planes {
