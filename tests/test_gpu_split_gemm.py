@@ -177,3 +177,20 @@ def test_sums_of_one_sign_are_not_biased(dev):
         e = (got - want) / want * 2.0 ** 24
         assert np.max(np.abs(e)) <= 12
         assert abs(e.mean()) <= 5 * 12 / np.sqrt(e.size)
+
+
+@pytest.mark.parametrize("power", [100, 112, 120])
+def test_gradients_of_tiny_values(dev, power):
+    """Output gradients down to 2^-120, whose lower parts bf16 cannot hold:
+    2-norm error of float32 sums, at most sqrt(terms) * 2^-24 of the sum's own
+    norm (9,800 terms in parts of 200 at most: 14 * 2^-24 = 9e-7), as 1e-6."""
+    rng = np.random.default_rng(9)
+    k, s = 3, 1
+    x = rng.standard_normal((200, 9, 9, 32)).astype(np.float32)
+    wt = rng.standard_normal((k * k * 32, 64)).astype(np.float32)
+    a = _patches(x, k, s)
+    dy = (rng.standard_normal((a.shape[0], 64)) * 2.0 ** -power).astype(np.float32)
+    dw, _, dx = _backward(dev, x, dy, wt, k, s, False)
+    g = dy.astype(np.float64)
+    for got, want in ((dw, a.T @ g), (dx, _scatter(g @ wt.astype(np.float64).T, x.shape, k, s))):
+        assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)

@@ -35,10 +35,13 @@
 //      barrier a stage.
 //
 // Infinities, NaN and values whose sums overflow do not survive the split
-// (inf - inf): a wavefront that finds a non-finite sum forms its tile again
-// with FP32 MFMA, whose results it then stores, so such inputs give what the
-// FP32 core gives.  Parts below bf16's smallest normal number (inputs under
-// 2^-110) may be lost, an absolute error under 2^-126 of the other operand.
+// (inf - inf), and operands under 2^-110 lose their lowest bits (bf16 ends at
+// 2^-133).  A wavefront that finds a non-finite sum, or no sum of kSplitTiny in
+// its tile, forms the tile again with FP32 MFMA, whose results it then stores,
+// so such inputs give what the FP32 core gives; what small operands lose beside
+// larger ones is under 2^-134 of the other operand.  A tile of exact zeros stays
+// (masked gradients are often zero throughout), so sums whose every operand
+// lies under 2^-134, below float32's normal range, may vanish.
 #pragma once
 
 #include "tile_gemm.hpp"
@@ -329,6 +332,9 @@ struct BStage<BN, FN, KB, NT, PERM, VB, false> {
 };
 
 constexpr int kSplitKB = 64;
+// With operands up to 2^16 on the other side and 2^12 terms, 2^-134 of them is
+// under 2^-24 of this.
+constexpr float kSplitTiny = 0x1p-80f;
 
 template <int WM, int FN, int NW, class LA, class LB, class EP>
 __global__ __launch_bounds__(64 * NW) void k_split(LA la, LB lb, EP ep, float* ws, int M, int N, int K, int kchunk,
@@ -456,6 +462,7 @@ __global__ __launch_bounds__(64 * NW) void k_split(LA la, LB lb, EP ep, float* w
   }
 
   bool finite = true;
+  float top = 0.f;
 #pragma unroll
   for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -464,8 +471,9 @@ __global__ __launch_bounds__(64 * NW) void k_split(LA la, LB lb, EP ep, float* w
       for (int r = 0; r < 4; ++r) {
         acc[i][j][r] += low[i][j][r];
         finite = finite && __builtin_isfinite(acc[i][j][r]);
+        top = fmaxf(top, fabsf(acc[i][j][r]));
       }
-  if (!__all(finite)) {
+  if (!__all(finite) || (__any(top > 0.f) && !__any(top >= kSplitTiny))) {
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
