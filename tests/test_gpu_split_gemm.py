@@ -78,9 +78,10 @@ def _backward(dev, x, dy, wt, k, s, u8, scale=1.0, mask=None, bank=None):
 
 
 # (batch, channels, size, out, kernel, stride): batches on both sides of each
-# rule's line, rows and columns one past a tile, input channels that are and
-# are not whole fragments of columns, strides whose residue classes differ.
-CONVS = [(166, 32, 8, 64, 3, 1), (167, 32, 8, 64, 3, 1), (400, 32, 7, 32, 2, 1), (251, 36, 9, 96, 5, 1),
+# rule's line (test_which_core_forms_a_gradient), rows and columns one past a
+# tile, input channels that are and are not whole fragments of columns, strides
+# whose residue classes differ.
+CONVS = [(301, 32, 8, 64, 3, 1), (302, 32, 8, 64, 3, 1), (166, 32, 8, 64, 3, 1), (167, 32, 8, 64, 3, 1), (400, 32, 7, 32, 2, 1), (251, 36, 9, 96, 5, 1),
          (110, 32, 20, 64, 4, 2), (700, 64, 5, 32, 3, 1), (170, 20, 14, 64, 2, 2), (130, 96, 11, 20, 3, 1)]
 
 
@@ -105,8 +106,9 @@ def test_convolution_gradients(dev, b, c, size, o, k, s, bank):
     assert np.all(np.abs(dx - want) <= _bound(k * k * o, magnitude))
 
 
-@pytest.mark.parametrize("b,c,h,w,o", [(15, 4, 84, 84, 32), (16, 4, 84, 84, 32), (25, 3, 100, 100, 16), (700, 1, 36, 36, 32),
-                                       (90, 4, 84, 52, 20), (97, 2, 84, 84, 64)])
+@pytest.mark.parametrize("b,c,h,w,o", [(15, 4, 84, 84, 32), (61, 4, 84, 84, 32), (62, 4, 84, 84, 32), (25, 3, 100, 100, 16),
+                                       (60, 3, 100, 100, 16), (700, 1, 36, 36, 32), (90, 4, 84, 52, 20),
+                                       (110, 4, 84, 52, 20), (97, 2, 84, 84, 64)])
 def test_frames_weight_gradient(dev, b, c, h, w, o):
     rng = np.random.default_rng(b)
     x = rng.integers(0, 256, (b, c, h, w), dtype=np.uint8)
@@ -145,6 +147,75 @@ def test_values_outside_the_split(dev, value):
             assert np.all(np.abs(got - want)[fine] <= _bound(terms, magnitude[fine]))
 
 
+class _Layer:
+    """One layer's operands on the device and its gradient entry points; the
+    gradients of a call under `fp32`, or by the rule that picks the core."""
+
+    def __init__(self, dev, b, c, size, o, k, s, u8=False, p=0):
+        from ttrl_amd.engine.tensor import to_device
+
+        rng = np.random.default_rng(b + size)
+        self.dev, self.dims = dev, (b, c, size, o, k, s, u8, p)
+        oh = (size + 2 * p - k) // s + 1
+        x = rng.integers(0, 256, (b, c, size, size), dtype=np.uint8) if u8 else \
+            rng.standard_normal((b, size, size, c)).astype(np.float32)
+        self.x = to_device(x, dev, x.dtype)
+        self.wt = to_device(rng.standard_normal((k * k * c, o)).astype(np.float32), dev)
+        self.dy = to_device(rng.standard_normal((b * oh * oh, o)).astype(np.float32), dev)
+
+    def geom(self, fp32):
+        from ttrl_amd import _lib
+
+        b, c, size, o, k, s, u8, p = self.dims
+        layout = _lib.LAYOUT_NCHW_U8 if u8 else _lib.LAYOUT_NHWC_F32
+        return C.byref(_lib.ConvGeom(b, c, size, size, o, k, s, p, layout | (_lib.CONV_FP32_ORDER if fp32 else 0)))
+
+    def _out(self, shape):
+        from ttrl_amd.engine.tensor import DeviceArray
+
+        return DeviceArray(self.dev, shape)
+
+    def weight(self, fp32):
+        dw, db = self._out(self.wt.shape), self._out((1, self.dims[3]))
+        self.dev.call("ttrl_conv2d_backward_weight", self.geom(fp32), self.x.vp, C.c_float(1.0), self.dy.vp, None, dw.vp,
+                      db.vp, C.c_float(0.0))
+        return dw.numpy()
+
+    def input(self, fp32):
+        dx = self._out(self.x.shape)
+        self.dev.call("ttrl_conv2d_backward_input", self.geom(fp32), self.dy.vp, None, self.wt.vp, dx.vp, None,
+                      C.c_float(1.0), C.c_float(0.0))
+        return dx.numpy()
+
+
+# Frames and float layers, and whether the split core forms their weight
+# gradient and their input gradient (None: there is none).
+CORES = [((32, 4, 84, 32, 8, 4, True), False, None),   # 105 M products
+         ((61, 4, 84, 32, 8, 4, True), False, None),   # 199.9 M
+         ((62, 4, 84, 32, 8, 4, True), True, None),
+         ((75, 3, 52, 32, 8, 4, True), False, None),   # 66 M
+         ((512, 3, 52, 32, 8, 4, True), True, None),   # a weight of 192 x 32 bytes' products
+         ((512, 1, 84, 32, 8, 4, True), False, None),  # 420 M, but a weight of 64 x 32
+         ((32, 32, 20, 64, 4, 2), False, False),       # 85 M; 100 tiles
+         ((64, 32, 20, 64, 4, 2), False, True),        # 170 M; 200 tiles
+         ((256, 32, 20, 64, 4, 2), True, True),
+         ((96, 64, 9, 64, 3, 1), False, False),        # 173 M; 122 tiles
+         ((128, 64, 9, 64, 3, 1), True, True),         # 231 M; 162 tiles
+         ((512, 16, 12, 32, 3, 1), False, True),       # 236 M, but a weight of 144 x 32; 576 tiles
+         ((300, 32, 18, 20, 4, 2), True, False),       # 20 outputs: dX reads 32 at a time
+         ((512, 32, 8, 32, 2, 2), False, True)]        # K 32; 256 tiles
+
+
+@pytest.mark.parametrize("dims,dw,dx", CORES)
+def test_which_core_forms_a_gradient(dev, dims, dw, dx):
+    """Sums on the two cores differ in their last bits, so whether a gradient
+    is the one under TTRL_CONV_FP32_ORDER shows which core formed it."""
+    layer = _Layer(dev, *dims)
+    assert np.array_equal(layer.weight(False), layer.weight(True)) == (not dw)
+    if dx is not None:
+        assert np.array_equal(layer.input(False), layer.input(True)) == (not dx)
+
+
 def test_short_sums_of_the_worst_operands(dev):
     """Sums of 32 products (one step of the core) of operands whose mantissa
     leaves most in the lower parts (0x00ffff).  In 2^-24 of the sum: 1 for the
@@ -152,9 +223,9 @@ def test_short_sums_of_the_worst_operands(dev):
     for adding the lower products' sum."""
     rng = np.random.default_rng(5)
     one = np.array([0x3F80FFFF], np.uint32).view(np.float32)[0]
-    x = np.ones((512, 8, 8, 32), np.float32)
-    wt = one * np.exp2(rng.integers(-3, 4, (4 * 32, 32))).astype(np.float32)
-    dy = one * np.exp2(rng.integers(-3, 4, (512 * 16, 32))).astype(np.float32)
+    x = np.ones((1600, 8, 8, 64), np.float32)
+    wt = one * np.exp2(rng.integers(-3, 4, (4 * 64, 32))).astype(np.float32)
+    dy = one * np.exp2(rng.integers(-3, 4, (1600 * 16, 32))).astype(np.float32)
     _, _, dx = _backward(dev, x, dy, wt, 2, 2, False)
     want = _scatter(dy.astype(np.float64) @ wt.astype(np.float64).T, x.shape, 2, 2)
     assert np.max(np.abs(dx - want) / want) <= 6 * 2.0 ** -24

@@ -151,20 +151,32 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 // of `kchunk`, as many as fill the device twice with 64-row tiles and as the
 // room for partials and kMaxDwSplits (whoever sums them reads them all)
 // allow.  splits 0: the FP32 core, for operands that do not fit (out channels
-// in whole float4s) and for fewer than kSplitPixels pixels, where a part is too
-// short to pay for more partials (third layer with its sum at 4,900 pixels:
-// FP32 13.7 us, split 15.0; at 6,272: 15.5 / 15.0).
+// in whole float4s) and for gradients too small to pay for more partials.  Two
+// lines, timed over first layers of 1 to 4 frames and float layers of 1 x 1 to
+// 5 x 5 kernels at 8 to 2,048 images (FP32 / split us):
+//   kSplitProducts, in products with the last tile's empty columns: first layer
+//     of 4 frames at 19,200 pixels (157 M) 13.6 / 13.7, at 25,600 (210 M) 16.2 /
+//     15.5; second layer at 5,184 (170 M) 13.7 / 14.9, at 7,776 (255 M) 17.9 /
+//     15.8; third at 4,704 (173 M) 13.8 / 15.4, at 9,408 (347 M) 20.8 / 17.5.
+//   kSplitArea, weight elements: a smaller weight has too few tiles for the
+//     parts that kMaxDwSplits allows.  144 x 32 at 51,200 pixels 19.5 / 24.3, at
+//     165,888 39.6 / 55.0; 192 x 32 at 41,472 21.4 / 22.0; 256 x 32 wins as above.
+//     Bytes take half the products: 192 x 32 of three frames at 73,728 pixels
+//     26.4 / 25.9, at 204,800 57.9 / 54.9, 64 x 32 at 294,912 39.8 / 74.7.
 constexpr int kMaxDwSplits = 64;
-constexpr int kSplitPixels = 6000;
+constexpr long kSplitProducts = 200'000'000;
+constexpr long kSplitArea = 8192, kSplitAreaU8 = 6144;
 struct DwSplit {
   SplitTile tile;
   int splits = 0, kchunk = 0;
 };
 inline DwSplit dw_split(const ConvGeo& g, const float* dy, int ones, long room) {
   DwSplit d;
-  if (g.fp32_order || g.O % 4 || g.M < kSplitPixels || !aligned16(dy) || gemm_force_set()) return d;
+  if (g.fp32_order || g.O % 4 || !aligned16(dy) || gemm_force_set()) return d;
   const int kp = g.C * g.KH * g.KW;
   d.tile = SplitTile{1, g.O > 32 ? 4 : 2};
+  const long area = long(kp) * ceil_div(g.O, 16 * d.tile.fn) * (16 * d.tile.fn);
+  if (area < (g.u8 ? kSplitAreaU8 : kSplitArea) || area * g.M < kSplitProducts) return d;
   const long tiles = long(ceil_div(kp, 64)) * ceil_div(g.O, 16 * d.tile.fn);
   const long stages = ceil_div(g.M, kSplitKB);
   const long most = std::min({room / (long(kp + ones) * g.O), long(kMaxDwSplits), stages});
