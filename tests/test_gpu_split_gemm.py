@@ -187,6 +187,20 @@ class _Layer:
                       C.c_float(1.0), C.c_float(0.0))
         return dx.numpy()
 
+    def both(self, bank=None):
+        """ttrl_conv2d_backward, or with a bank ttrl_conv2d_backward_deferred
+        (no dW: its partials stay in the bank) -> dW, dX."""
+        from ttrl_amd import _lib
+
+        dw, db, dx = self._out(self.wt.shape), self._out((1, self.dims[3])), self._out(self.x.shape)
+        args = (self.geom(False), self.x.vp, C.c_float(1.0), self.dy.vp, None, self.wt.vp, dw.vp, db.vp)
+        if bank is None:
+            self.dev.call("ttrl_conv2d_backward", *args, C.c_float(0.0), dx.vp, None, C.c_float(0.0))
+            return dw.numpy(), dx.numpy()
+        src = _lib.GradSource()
+        self.dev.call("ttrl_conv2d_backward_deferred", *args, dx.vp, None, C.c_float(0.0), bank, C.byref(src))
+        return None, dx.numpy()
+
 
 # Frames and float layers, and whether the split core forms their weight
 # gradient and their input gradient (None: there is none).
@@ -197,6 +211,8 @@ CORES = [((32, 4, 84, 32, 8, 4, True), False, None),   # 105 M products
          ((512, 3, 52, 32, 8, 4, True), True, None),   # a weight of 192 x 32 bytes' products
          ((512, 1, 84, 32, 8, 4, True), False, None),  # 420 M, but a weight of 64 x 32
          ((32, 32, 20, 64, 4, 2), False, False),       # 85 M; 100 tiles
+         ((47, 32, 20, 64, 4, 2), False, False),       # 125 M; 148 tiles
+         ((48, 32, 20, 64, 4, 2), False, True),        # 150 tiles
          ((64, 32, 20, 64, 4, 2), False, True),        # 170 M; 200 tiles
          ((256, 32, 20, 64, 4, 2), True, True),
          ((96, 64, 9, 64, 3, 1), False, False),        # 173 M; 122 tiles
@@ -214,6 +230,26 @@ def test_which_core_forms_a_gradient(dev, dims, dw, dx):
     assert np.array_equal(layer.weight(False), layer.weight(True)) == (not dw)
     if dx is not None:
         assert np.array_equal(layer.input(False), layer.input(True)) == (not dx)
+
+
+@pytest.mark.parametrize("dims,dw,dx", [row for row in CORES if row[2] or (row[1] and row[2] is not None)])
+@pytest.mark.parametrize("bank", [None, 2])
+def test_both_gradients_choose_their_cores_apart(dev, dims, dw, dx, bank):
+    """The call for both gradients: what the split core forms for a call of its
+    own it forms there too, bit for bit, except where the call has timed one
+    launch of both on the FP32 core as faster."""
+    layer = _Layer(dev, *dims)
+    both_dw, both_dx = layer.both(bank)
+    b, c, size, o, k, s = dims
+    key = f"ttrl_conv2d_backward:pair|0|{b}|{c}|{size}|{size}|{o}|{k}|{k}|{s}|0|0|0|{int(bank is not None)}|split"
+    plan = [row.split("\t")[0].split()[0] for row in dev.export_plans().splitlines() if row.endswith(key)]
+    assert len(plan) == 1
+    separate = plan[0] == "0"
+    if dx:
+        assert np.array_equal(both_dx, layer.input(False)) == separate
+    if dw and bank is None:
+        assert np.array_equal(both_dw, layer.weight(False)) == separate
+    assert separate or not (dw and dx)  # both well past the lines
 
 
 def test_short_sums_of_the_worst_operands(dev):

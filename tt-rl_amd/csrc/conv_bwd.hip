@@ -3,7 +3,8 @@
 // weight gradient and the first launch of the input gradient (its first
 // four residue classes) can run as one paired launch, which saves a launch
 // but makes both problems take one tile shape; at large batches the two as
-// separate launches, each with its own tile shape, are faster.  Both calls
+// separate launches, each with its own tile shape, are faster, and a gradient
+// large enough for the split core (conv_split.hpp) takes a launch of its own.  Both calls
 // (the plain one and the one that leaves the weight gradient's split-K
 // partials to the optimizer step) time the two ways once per geometry
 // (outside capture, on scratch outputs) and keep the faster for the context.
@@ -39,16 +40,18 @@ int conv_backward_pair(ttrl_ctx* ctx, const ConvGeo& g, const void* x, float x_s
   return rc;
 }
 
-// The two gradients as separate launches, each GEMM with its own plan; bank
-// as for conv_backward_pair.
+// The two gradients as separate launches, each on the core that
+// ttrl_conv2d_backward_weight and ttrl_conv2d_backward_input would take, a
+// GEMM of the FP32 core with its own plan; bank as for conv_backward_pair.
 template <int MODE>
-int conv_backward_split(ttrl_ctx* ctx, const ConvGeo& g, const void* x, float x_scale, const float* dy,
-                        const float* wt, float* dwt, float* db, float beta_w, float* dx, const float* xmask,
-                        float beta_x, long reserved, float* bank = nullptr, ttrl_grad_source* out = nullptr) {
+int conv_backward_separate(ttrl_ctx* ctx, const ConvGeo& g, const void* x, float x_scale, const float* dy,
+                           const float* wt, float* dwt, float* db, float beta_w, float* dx, const float* xmask,
+                           float beta_x, long reserved, float* bank = nullptr, ttrl_grad_source* out = nullptr) {
   constexpr unsigned kDw = MODE == kPatchGeneral ? kConvGeneralCfgs : kConvDwCfgs;
   const ConvDwProblem<MODE> w = conv_dw_problem<MODE>(g, x, x_scale, dy, dwt, db, beta_w);
   int rc = TTRL_OK;
-  if (bank) {
+  if (conv_dw_split(ctx, w, g, x, x_scale, dy, dwt, db, reserved, bank, out, "ttrl_conv2d_backward", &rc)) {
+  } else if (bank) {
     GemmPlan plan{};
     rc = run_gemm_deferred<kDw>(ctx, w.la, w.lb, w.ep, w.q.M, w.q.N, w.q.K, 1, "ttrl_conv2d_backward_deferred",
                                 &plan, bank, kGradBankFloats);
@@ -56,15 +59,12 @@ int conv_backward_split(ttrl_ctx* ctx, const ConvGeo& g, const void* x, float x_
   } else {
     rc = run_gemm<kDw>(ctx, w.la, w.lb, w.ep, w.q.M, w.q.N, w.q.K, 1, "ttrl_conv2d_backward", reserved);
   }
-  for (int c0 = 0; c0 < g.S * g.S && rc == TTRL_OK; c0 += kMaxGroups) {
-    const ConvDxProblem d = conv_dx_problem(g, c0, dy, wt, dx, xmask, x_scale, beta_x);
-    rc = run_gemm<kConvDxCfgs>(ctx, d.la, d.lb, d.ep, d.q.M, d.q.N, d.q.K, d.q.groups, "ttrl_conv2d_backward",
-                               reserved);
-  }
-  return rc;
+  if (rc != TTRL_OK) return rc;
+  return conv_dx(ctx, g, dy, wt, dx, xmask, x_scale, beta_x, reserved, "ttrl_conv2d_backward");
 }
 
-// Whether the paired launch is the faster way for this geometry.  Kept in
+// Whether the paired launch is the faster way for this geometry; `split`:
+// against separate launches of which some take the split core.  Kept in
 // the context's plan table as {cfg 1: pair, 0: separate; 0, 0, 0, 1, 0}, so
 // it is exported and imported with the GEMM plans and every later call,
 // eager or captured, takes the same path; an entry of any other form (an
@@ -77,10 +77,10 @@ inline bool is_pair_choice(const GemmPlan& p) {
 }
 template <int MODE>
 bool pair_is_faster(ttrl_ctx* ctx, const ConvGeo& g, const void* x, float x_scale, const float* dy,
-                    const float* wt, const float* xmask, long reserved, float* bank) {
+                    const float* wt, const float* xmask, long reserved, float* bank, bool split) {
   char keybuf[192];
-  snprintf(keybuf, sizeof(keybuf), "ttrl_conv2d_backward:pair|%d|%d|%d|%d|%d|%d|%d|%d|%d|%d|%ld|%d|%d", MODE, g.B,
-           g.C, g.H, g.W, g.O, g.KH, g.KW, g.S, g.P, reserved, xmask ? 1 : 0, bank ? 1 : 0);
+  snprintf(keybuf, sizeof(keybuf), "ttrl_conv2d_backward:pair|%d|%d|%d|%d|%d|%d|%d|%d|%d|%d|%ld|%d|%d%s", MODE, g.B,
+           g.C, g.H, g.W, g.O, g.KH, g.KW, g.S, g.P, reserved, xmask ? 1 : 0, bank ? 1 : 0, split ? "|split" : "");
   const std::string key(keybuf);
   if (const GemmPlan* hit = ctx_plan_find(ctx, key))
     if (is_pair_choice(*hit)) return hit->cfg == 1;
@@ -93,19 +93,21 @@ bool pair_is_faster(ttrl_ctx* ctx, const ConvGeo& g, const void* x, float x_scal
       float *sw = out, *sb = out + nw, *sx = out + nw + g.O;
       hipStream_t st = stream_of(ctx);
       int rc = TTRL_OK;
+      ConvGeo tg = g;
+      if (!split) tg.fp32_order = 1;  // the scratch outputs' alignment does not bring in the split core
       ttrl_grad_source src{};  // the deferred form's partials go to the bank the real call then overwrites
       auto paired = [&] {
-        if (rc == TTRL_OK) rc = conv_backward_pair<MODE>(ctx, g, x, x_scale, dy, wt, sw, sb, 0.f, sx, xmask, 0.f,
+        if (rc == TTRL_OK) rc = conv_backward_pair<MODE>(ctx, tg, x, x_scale, dy, wt, sw, sb, 0.f, sx, xmask, 0.f,
                                                          reserved, bank, &src);
       };
-      auto split = [&] {
-        if (rc == TTRL_OK) rc = conv_backward_split<MODE>(ctx, g, x, x_scale, dy, wt, sw, sb, 0.f, sx, xmask, 0.f,
-                                                          reserved, bank, &src);
+      auto separate = [&] {
+        if (rc == TTRL_OK) rc = conv_backward_separate<MODE>(ctx, tg, x, x_scale, dy, wt, sw, sb, 0.f, sx, xmask,
+                                                             0.f, reserved, bank, &src);
       };
       paired();  // first runs: each GEMM's own plan is tuned here
-      split();
+      separate();
       const float tp = rc == TTRL_OK ? time_best_of(e0, e1, st, paired) : -1.f;
-      const float ts = rc == TTRL_OK ? time_best_of(e0, e1, st, split) : -1.f;
+      const float ts = rc == TTRL_OK ? time_best_of(e0, e1, st, separate) : -1.f;
       if (tp > 0.f && ts > 0.f) pair = tp <= ts;
       if (gemm_tuning_log())
         fprintf(stderr, "[ttrl gemm tune] conv2d backward B=%d C=%d %dx%d O=%d k=%d s=%d: pair %.2f us, "
@@ -123,28 +125,18 @@ template <int MODE>
 int conv_backward_chosen(ttrl_ctx* ctx, const ConvGeo& g, const void* x, float x_scale, const float* dy,
                          const float* wt, float* dwt, float* db, float beta_w, float* dx, const float* xmask,
                          float beta_x, long reserved, float* bank = nullptr, ttrl_grad_source* out = nullptr) {
-  if constexpr (MODE != kPatchGeneral) {
-    // Both gradients on the split core, where it takes both: a launch each.
-    const ConvDxProblem d0 = conv_dx_problem(g, 0, dy, wt, dx, xmask, x_scale, beta_x);
-    int rc = TTRL_OK;
-    if (dx_split(g, d0).wm &&
-        conv_dw_split(ctx, conv_dw_problem<MODE>(g, x, x_scale, dy, dwt, db, beta_w), g, x, x_scale, dy, dwt, db,
-                      reserved, bank, out, "ttrl_conv2d_backward", &rc)) {
-      for (int c0 = 0; c0 < g.S * g.S && rc == TTRL_OK; c0 += kMaxGroups) {
-        const ConvDxProblem d = conv_dx_problem(g, c0, dy, wt, dx, xmask, x_scale, beta_x);
-        const SplitTile t = dx_split(g, d);
-        rc = t.wm ? run_dx_split(ctx, t, d, "ttrl_conv2d_backward")
-                  : run_gemm<kConvDxCfgs>(ctx, d.la, d.lb, d.ep, d.q.M, d.q.N, d.q.K, d.q.groups,
-                                          "ttrl_conv2d_backward", reserved);
-      }
-      return rc;
-    }
-  }
-  if (pair_is_faster<MODE>(ctx, g, x, x_scale, dy, wt, xmask, reserved, bank))
+  // A gradient on the split core is a launch of its own, a pair is of two GEMMs
+  // of the FP32 core: where the split core takes a gradient the choice is timed
+  // too, since near its lines the faster way hangs on how full the FP32 core's
+  // last waves are (updates of a DQN, pair / split us: 64 images of 84 x 84 180.6 /
+  // 176.2, 48 of 100 x 100 198.7 / 202.0).
+  const bool split = conv_dw_splits<MODE>(ctx, g, dy, db, reserved, bank).splits ||
+                     dx_on_split(g, conv_dx_problem(g, 0, dy, wt, dx, xmask, x_scale, beta_x));
+  if (pair_is_faster<MODE>(ctx, g, x, x_scale, dy, wt, xmask, reserved, bank, split))
     return conv_backward_pair<MODE>(ctx, g, x, x_scale, dy, wt, dwt, db, beta_w, dx, xmask, beta_x, reserved, bank,
                                     out);
-  return conv_backward_split<MODE>(ctx, g, x, x_scale, dy, wt, dwt, db, beta_w, dx, xmask, beta_x, reserved, bank,
-                                   out);
+  return conv_backward_separate<MODE>(ctx, g, x, x_scale, dy, wt, dwt, db, beta_w, dx, xmask, beta_x, reserved, bank,
+                                      out);
 }
 
 }  // namespace

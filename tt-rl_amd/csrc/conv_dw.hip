@@ -12,16 +12,14 @@ int conv_backward_weight_mode(ttrl_ctx* ctx, const ConvGeo& g, const void* x, fl
                               float* dwt, float* db, float beta, long reserved, float* bank = nullptr,
                               ttrl_grad_source* out = nullptr) {
   const ConvDwProblem<MODE> p = conv_dw_problem<MODE>(g, x, x_scale, dy, dwt, db, beta);
-  if constexpr (MODE != kPatchGeneral) {
-    int rc = TTRL_OK;
-    if (conv_dw_split(ctx, p, g, x, x_scale, dy, dwt, db, reserved, bank, out, "ttrl_conv2d_backward_weight", &rc))
-      return rc;
-  }
+  int rc = TTRL_OK;
+  if (conv_dw_split(ctx, p, g, x, x_scale, dy, dwt, db, reserved, bank, out, "ttrl_conv2d_backward_weight", &rc))
+    return rc;
   if (!bank)
     return run_gemm<CFGS>(ctx, p.la, p.lb, p.ep, p.q.M, p.q.N, p.q.K, 1, "ttrl_conv2d_backward_weight", reserved);
   GemmPlan plan{};
-  const int rc = run_gemm_deferred<CFGS>(ctx, p.la, p.lb, p.ep, p.q.M, p.q.N, p.q.K, 1,
-                                         "ttrl_conv2d_backward_weight_deferred", &plan, bank, kGradBankFloats);
+  rc = run_gemm_deferred<CFGS>(ctx, p.la, p.lb, p.ep, p.q.M, p.q.N, p.q.K, 1, "ttrl_conv2d_backward_weight_deferred",
+                               &plan, bank, kGradBankFloats);
   if (rc == TTRL_OK) *out = conv_dw_source(g, x_scale, dwt, db, bank, plan);
   return rc;
 }

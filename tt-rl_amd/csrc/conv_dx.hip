@@ -21,17 +21,7 @@ int ttrl_conv2d_backward_input(ttrl_ctx* ctx, const ttrl_conv_geom* geom, const 
     dy = relu_mask_into_workspace(ctx, dy, ymask, long(g.M) * g.O, 0, 1, &reserved, &rc);
     if (rc) return rc;
   }
-  for (int c0 = 0; c0 < g.S * g.S; c0 += kMaxGroups) {
-    const ConvDxProblem p = conv_dx_problem(g, c0, dy, wt, dx, xmask, x_scale, beta);
-    const SplitTile t = dx_split(g, p);
-    if (t.wm)
-      rc = run_dx_split(ctx, t, p, "ttrl_conv2d_backward_input");
-    else
-      rc = run_gemm<kConvDxCfgs>(ctx, p.la, p.lb, p.ep, p.q.M, p.q.N, p.q.K, p.q.groups, "ttrl_conv2d_backward_input",
-                                 reserved);
-    if (rc) return rc;
-  }
-  return TTRL_OK;
+  return conv_dx(ctx, g, dy, wt, dx, xmask, x_scale, beta, reserved, "ttrl_conv2d_backward_input");
 }
 
 }  // extern "C"

@@ -151,7 +151,7 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 // of `kchunk`, as many as fill the device twice with 64-row tiles and as the
 // room for partials and kMaxDwSplits (whoever sums them reads them all)
 // allow.  splits 0: the FP32 core, for operands that do not fit (out channels
-// in whole float4s) and for gradients too small to pay for more partials.  Two
+// in whole float4s) and for gradients too small to pay for more partials.  The
 // lines, timed over first layers of 1 to 4 frames and float layers of 1 x 1 to
 // 5 x 5 kernels at 8 to 2,048 images (FP32 / split us):
 //   kSplitProducts, in products with the last tile's empty columns: first layer
@@ -163,20 +163,27 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 //     165,888 39.6 / 55.0; 192 x 32 at 41,472 21.4 / 22.0; 256 x 32 wins as above.
 //     Bytes take half the products: 192 x 32 of three frames at 73,728 pixels
 //     26.4 / 25.9, at 204,800 57.9 / 54.9, 64 x 32 at 294,912 39.8 / 74.7.
+//   kSplitBank, where the partials stay in a bank and the FP32 core saves no
+//     launch: the second layer's partials at 5,184 pixels (170 M) 9.6 / 8.6, the
+//     third's at 4,704 (173 M) 9.6 / 8.7.  Of bytes (updates of a DQN, 24 to 100
+//     images of 52 to 84): at 59 M 122 / 120, at 67 M 112.3 / 111, at 88 M 128 / 124,
+//     at 105 M equal, the optimizer step reading twice the parts; at 21 M 84 / 87, at
+//     28 M 86 / 88.
 constexpr int kMaxDwSplits = 64;
-constexpr long kSplitProducts = 200'000'000;
+constexpr long kSplitProducts = 200'000'000, kSplitBank = 150'000'000, kSplitBankU8 = 40'000'000;
 constexpr long kSplitArea = 8192, kSplitAreaU8 = 6144;
 struct DwSplit {
   SplitTile tile;
   int splits = 0, kchunk = 0;
 };
-inline DwSplit dw_split(const ConvGeo& g, const float* dy, int ones, long room) {
+inline DwSplit dw_split(const ConvGeo& g, const float* dy, int ones, long room, bool bank) {
   DwSplit d;
   if (g.fp32_order || g.O % 4 || !aligned16(dy) || gemm_force_set()) return d;
   const int kp = g.C * g.KH * g.KW;
   d.tile = SplitTile{1, g.O > 32 ? 4 : 2};
   const long area = long(kp) * ceil_div(g.O, 16 * d.tile.fn) * (16 * d.tile.fn);
-  if (area < (g.u8 ? kSplitAreaU8 : kSplitArea) || area * g.M < kSplitProducts) return d;
+  if (area < (g.u8 ? kSplitAreaU8 : kSplitArea)) return d;
+  if (area * g.M < (!bank ? kSplitProducts : g.u8 ? kSplitBankU8 : kSplitBank)) return d;
   const long tiles = long(ceil_div(kp, 64)) * ceil_div(g.O, 16 * d.tile.fn);
   const long stages = ceil_div(g.M, kSplitKB);
   const long most = std::min({room / (long(kp + ones) * g.O), long(kMaxDwSplits), stages});
@@ -203,47 +210,82 @@ inline int run_dw_split(ttrl_ctx* ctx, const DwSplit& d, const ConvGeo& g, const
   return run_split(ctx, d.tile, la, lb, ep, ep.M, g.O, g.M, 1, name, ones, part, d.splits, d.kchunk);
 }
 
+// dw_split for a layer whose partials go to `bank`, or to the workspace past
+// `reserved` floats at its end (bank null); never for the general patch path.
+template <int MODE>
+inline DwSplit conv_dw_splits(ttrl_ctx* ctx, const ConvGeo& g, const float* dy, const float* db, long reserved,
+                              const float* bank, float** part = nullptr) {
+  if constexpr (MODE == kPatchGeneral) return DwSplit{};
+  long wsf = kGradBankFloats;
+  float* to = const_cast<float*>(bank);
+  if (!to) {
+    to = ctx_workspace(ctx, &wsf);
+    wsf -= reserved;
+  }
+  if (part) *part = to;
+  return dw_split(g, dy, db ? 1 : 0, wsf, bank != nullptr);
+}
+
 // The weight gradient on the split core, if it takes it: its partials left in
 // `bank` and described by *out (bank not null), or summed from the workspace.
 template <int MODE>
 inline bool conv_dw_split(ttrl_ctx* ctx, const ConvDwProblem<MODE>& p, const ConvGeo& g, const void* x, float x_scale,
                           const float* dy, float* dwt, float* db, long reserved, float* bank, ttrl_grad_source* out,
                           const char* name, int* rc) {
-  long wsf = kGradBankFloats;
-  float* part = bank;
-  if (!part) {
-    part = ctx_workspace(ctx, &wsf);
-    wsf -= reserved;
-  }
-  const int ones = db ? 1 : 0;
-  const DwSplit d = dw_split(g, dy, ones, wsf);
-  if (!d.splits) return false;
-  *rc = run_dw_split<MODE == kPatchU8Word>(ctx, d, g, x, dy, ones, part, name);
-  if (*rc != TTRL_OK) return true;
-  if (bank) {
-    GemmPlan plan{};
-    plan.splits = d.splits;
-    *out = conv_dw_source(g, x_scale, dwt, db, part, plan);
+  if constexpr (MODE == kPatchGeneral) {
+    return false;
+  } else {
+    float* part = nullptr;
+    const DwSplit d = conv_dw_splits<MODE>(ctx, g, dy, db, reserved, bank, &part);
+    if (!d.splits) return false;
+    *rc = run_dw_split<MODE == kPatchU8Word>(ctx, d, g, x, dy, db ? 1 : 0, part, name);
+    if (*rc != TTRL_OK) return true;
+    if (bank) {
+      GemmPlan plan{};
+      plan.splits = d.splits;
+      *out = conv_dw_source(g, x_scale, dwt, db, part, plan);
+      return true;
+    }
+    FDiv dn;
+    dn.set(p.q.N);
+    const unsigned blocks = std::min(2048u, unsigned(long(p.q.M) * p.q.N / 256 + 1));
+    hipLaunchKernelGGL((k_splitk_reduce<EpStore>), dim3(blocks, 1), dim3(256), 0, stream_of(ctx), part, p.ep, p.q.M,
+                       p.q.N, d.splits, dn);
+    *rc = check_launch(name);
     return true;
   }
-  FDiv dn;
-  dn.set(p.q.N);
-  const unsigned blocks = std::min(2048u, unsigned(long(p.q.M) * p.q.N / 256 + 1));
-  hipLaunchKernelGGL((k_splitk_reduce<EpStore>), dim3(blocks, 1), dim3(256), 0, stream_of(ctx), part, p.ep, p.q.M, p.q.N,
-                     d.splits, dn);
-  *rc = check_launch(name);
-  return true;
 }
 
-// Whether the split core runs the input gradient of the classes of `p`.
-inline SplitTile dx_split(const ConvGeo& g, const ConvDxProblem& p) {
-  if (g.fp32_order || g.O % 32 || g.C % 4 || gemm_force_set() || !aligned16(p.la.dy) || !aligned16(p.lb.wt) || !aligned16(p.ep.dx) ||
-      !aligned16(p.ep.xmask))
-    return SplitTile{};
-  return split_tile(p.q.M, p.q.N, p.q.groups);
+// Whether the split core forms a layer's input gradient; `first` its problem of
+// the first residue classes, which are the most and the largest.  The lines
+// were timed over 1 x 1 to 5 x 5 kernels at 8 to 512 images.  Under kSplitTiles
+// the FP32 core's smaller tiles fill the device better (FP32 / split us: the
+// third Nature-CNN layer's at 122 tiles 13.3 / 15.6, at 162 19.3 / 15.7; 3 x 3 on
+// 32 channels at 128 9.4 / 10.7, at 192 12.9 / 11.0; of 32 columns, 5 x 5 at 100
+// 24.4 / 26.3, at 200 40.8 / 34.9).  K plays no part down to 32 (half a stage of
+// zeros): 1 x 1 at 256 7.0 / 6.6, 2 x 2 in strides of 2 at 576 12.0 / 9.6.
+constexpr long kSplitTiles = 150;
+inline bool dx_on_split(const ConvGeo& g, const ConvDxProblem& first) {
+  return !g.fp32_order && g.O % 32 == 0 && g.C % 4 == 0 && !gemm_force_set() && aligned16(first.la.dy) &&
+         aligned16(first.lb.wt) && aligned16(first.ep.dx) && aligned16(first.ep.xmask) &&
+         split_tiles(first.q.M, first.q.N, first.q.groups) >= kSplitTiles;
 }
-inline int run_dx_split(ttrl_ctx* ctx, const SplitTile& t, const ConvDxProblem& p, const char* name) {
-  return run_split(ctx, t, SaConvDx{p.la}, SbConvDx{p.lb}, SeConvDx{p.ep}, p.q.M, p.q.N, p.q.K, p.q.groups, name);
+
+// The input gradient, kMaxGroups residue classes a launch, all on one core.
+inline int conv_dx(ttrl_ctx* ctx, const ConvGeo& g, const float* dy, const float* wt, float* dx, const float* xmask,
+                   float x_scale, float beta, long reserved, const char* name) {
+  bool split = false;
+  int rc = TTRL_OK;
+  for (int c0 = 0; c0 < g.S * g.S && rc == TTRL_OK; c0 += kMaxGroups) {
+    const ConvDxProblem p = conv_dx_problem(g, c0, dy, wt, dx, xmask, x_scale, beta);
+    if (c0 == 0) split = dx_on_split(g, p);
+    if (split)
+      rc = run_split(ctx, split_tile(p.q.M, p.q.N, p.q.groups), SaConvDx{p.la}, SbConvDx{p.lb}, SeConvDx{p.ep}, p.q.M,
+                     p.q.N, p.q.K, p.q.groups, name);
+    else
+      rc = run_gemm<kConvDxCfgs>(ctx, p.la, p.lb, p.ep, p.q.M, p.q.N, p.q.K, p.q.groups, name, reserved);
+  }
+  return rc;
 }
 
 }  // namespace ttrl

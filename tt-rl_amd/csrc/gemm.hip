@@ -114,9 +114,13 @@ SplitTile split_tile(long M, long N, long groups) {
   t.fn = N > 32 ? 4 : 2;
   const long cols = ceil_div(N, 16 * t.fn) * groups;
   const long t64 = ceil_div(M, 64) * cols, t128 = ceil_div(M, 128) * cols;
-  if (t64 * t.fn / 4 < kSplitTiles) return SplitTile{};
   t.wm = double(ceil_div(t128, 256)) <= 0.55 * double(ceil_div(t64, 256)) ? 2 : 1;
   return t;
+}
+
+long split_tiles(long M, long N, long groups) {
+  const int fn = split_tile(M, N, groups).fn;
+  return long(ceil_div(M, 64)) * ceil_div(N, 16 * fn) * groups * fn / 4;
 }
 
 bool gemm_force_set() {

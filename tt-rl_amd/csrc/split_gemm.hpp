@@ -567,24 +567,16 @@ __global__ __launch_bounds__(64 * NW) void k_split(LA la, LB lb, EP ep, float* w
 
 // ---------------------------------------------------------------- host ---
 
-// Whether a GEMM of these extents goes to the split core, and its tile: rows
-// of a workgroup (64 or 128; wm = 1, 2 fragments a wavefront) by 16 fn
-// columns.  Both lines were timed on convolution input gradients (1 x 1 to 5 x 5
-// kernels, 8 to 512 images).  Under kSplitTiles workgroups of 64 x 64, those of
-// 32 columns counted half, the FP32 core's smaller tiles fill the device better
-// (FP32 / split us: the third Nature-CNN layer's at 122 13.3 / 15.6, at 162 19.3 /
-// 15.7; 3 x 3 on 32 channels at 128 9.4 / 10.7, at 192 12.9 / 11.0; of 32 columns,
-// the second layer's at 200 7.7 / 7.9, at 400 11.1 / 10.1, 5 x 5 at 200 24.4 / 26.3,
-// at 400 40.8 / 34.9).  K plays no part down to 32 (half a stage of zeros): 1 x 1 at
-// 512 7.0 / 6.6, 2 x 2 in strides of 2 at 1,152 12.0 / 9.6.  Of the two heights the
-// one with the shorter last wave of workgroups, 64 rows costing 0.55 of 128 (third
-// layer at batch 512, 648 tiles of 64 or 324 of 128: 27.9 / 30.1 us; second layer,
-// 3200 or 1600: 37.6 / 36.2).
+// The split core's tile for a GEMM: rows of a workgroup (64 or 128; wm = 1, 2
+// fragments a wavefront) by 16 fn columns.  Of the two heights the one with the
+// shorter last wave of workgroups, 64 rows costing 0.55 of 128 (third Nature-CNN
+// layer's input gradient at batch 512, 648 tiles of 64 or 324 of 128: 27.9 / 30.1
+// us; second layer's, 3200 or 1600: 37.6 / 36.2).
 struct SplitTile {
-  int wm = 0, fn = 0;  // wm 0: the FP32 core
+  int wm = 0, fn = 0;
 };
-constexpr long kSplitTiles = 150;
 SplitTile split_tile(long M, long N, long groups);
+long split_tiles(long M, long N, long groups);  // its 64 x 64 tiles, those of 32 columns counted half
 
 // splits > 1: partials [groups][splits][M + ones][N] to ws.
 template <class LA, class LB, class EP>
