@@ -67,6 +67,7 @@ struct SbConvDx {
 
 // Input-gradient epilogue (EpConvDx); C a multiple of the columns a lane stores.
 struct SeConvDx {
+  static constexpr bool PARTIALS = false;
   EpConvDx src;
   struct Bound {
     EpConvDx::Bound b;
@@ -78,16 +79,12 @@ struct SeConvDx {
       const int ih = b.ih0 + b.S * i, iw = b.iw0 + b.S * j;
       return r < b.rows && c < b.C ? uint32_t(((n * b.H + ih) * b.W + iw) * b.C + c) * 4u : kBad;
     }
-    template <int FN>
-    __device__ __forceinline__ FVec<FN> bias(int) const { return FVec<FN>(0.f); }
     __device__ __forceinline__ float alpha() const { return b.alpha; }
     __device__ __forceinline__ float beta() const { return b.beta; }
-    __device__ __forceinline__ bool relu() const { return false; }
     __device__ __forceinline__ bool masked() const { return b.has_xm; }
     __device__ __forceinline__ bool accumulates() const { return b.beta != 0.f; }
   };
   __device__ __forceinline__ int rows(int grp) const { return src.rows(grp); }
-  __device__ __forceinline__ void store_sum(int, int, float) const {}
   __device__ __forceinline__ Bound bind(int grp) const {
     const EpConvDx::Bound b = src.bound(grp);
     return Bound{b, b.rdx, b.rxm};
@@ -173,18 +170,17 @@ constexpr int kMaxDwSplits = 64;
 constexpr long kSplitProducts = 200'000'000, kSplitBank = 150'000'000, kSplitBankU8 = 40'000'000;
 constexpr long kSplitArea = 8192, kSplitAreaU8 = 6144;
 struct DwSplit {
-  SplitTile tile;
-  int splits = 0, kchunk = 0;
+  int fn = 0, splits = 0, kchunk = 0;
 };
 inline DwSplit dw_split(const ConvGeo& g, const float* dy, int ones, long room, bool bank) {
   DwSplit d;
   if (g.fp32_order || g.O % 4 || !aligned16(dy) || gemm_force_set()) return d;
   const int kp = g.C * g.KH * g.KW;
-  d.tile = SplitTile{1, g.O > 32 ? 4 : 2};
-  const long area = long(kp) * ceil_div(g.O, 16 * d.tile.fn) * (16 * d.tile.fn);
+  d.fn = g.O > 32 ? 4 : 2;
+  const long area = long(kp) * ceil_div(g.O, 16 * d.fn) * (16 * d.fn);
   if (area < (g.u8 ? kSplitAreaU8 : kSplitArea)) return d;
   if (area * g.M < (!bank ? kSplitProducts : g.u8 ? kSplitBankU8 : kSplitBank)) return d;
-  const long tiles = long(ceil_div(kp, 64)) * ceil_div(g.O, 16 * d.tile.fn);
+  const long tiles = long(ceil_div(kp, 64)) * ceil_div(g.O, 16 * d.fn);
   const long stages = ceil_div(g.M, kSplitKB);
   const long most = std::min({room / (long(kp + ones) * g.O), long(kMaxDwSplits), stages});
   const long want = std::min(most, std::max(2L, 512 / tiles));
@@ -204,10 +200,10 @@ inline int run_dw_split(ttrl_ctx* ctx, const DwSplit& d, const ConvGeo& g, const
   lb.p[0] = dy;
   lb.ld = lb.rows = g.O;
   lb.K = g.M;
-  SeStore ep;  // the partials' reader applies the epilogue
-  ep.M = g.C * g.KH * g.KW;
-  ep.N = g.O;
-  return run_split(ctx, d.tile, la, lb, ep, ep.M, g.O, g.M, 1, name, ones, part, d.splits, d.kchunk);
+  const int M = g.C * g.KH * g.KW;
+  const SePartials ep{M};
+  if (d.fn == 4) return launch_split<1, 4>(ctx, la, lb, ep, M, g.O, g.M, 1, name, ones, part, d.splits, d.kchunk);
+  return launch_split<1, 2>(ctx, la, lb, ep, M, g.O, g.M, 1, name, ones, part, d.splits, d.kchunk);
 }
 
 // dw_split for a layer whose partials go to `bank`, or to the workspace past
@@ -280,8 +276,7 @@ inline int conv_dx(ttrl_ctx* ctx, const ConvGeo& g, const float* dy, const float
     const ConvDxProblem p = conv_dx_problem(g, c0, dy, wt, dx, xmask, x_scale, beta);
     if (c0 == 0) split = dx_on_split(g, p);
     if (split)
-      rc = run_split(ctx, split_tile(p.q.M, p.q.N, p.q.groups), SaConvDx{p.la}, SbConvDx{p.lb}, SeConvDx{p.ep}, p.q.M,
-                     p.q.N, p.q.K, p.q.groups, name);
+      rc = run_split(ctx, SaConvDx{p.la}, SbConvDx{p.lb}, SeConvDx{p.ep}, p.q.M, p.q.N, p.q.K, p.q.groups, name);
     else
       rc = run_gemm<kConvDxCfgs>(ctx, p.la, p.lb, p.ep, p.q.M, p.q.N, p.q.K, p.q.groups, name, reserved);
   }

@@ -98,13 +98,14 @@ __device__ __forceinline__ f32x4 mfma_bf16(const u32x4& a, const u32x4& b, const
 
 // ---------------------------------------------------------- A operands ---
 //
-// live(g) as for the FP32 core's loaders.  A step is 32 k; K is a multiple
-// of 32.  row(m, lg): the address part of one output row for lane group lg;
-// kbase(k0): of the step from k0 (wave-uniform, any k0: past K it makes
-// every address out of range); issue: starts a lane's loads; resolve: its 8
-// values.  With PERM lane group lg holds k = 4 lg .. 4 lg + 3 and 16 + 4 lg ..
-// of the step, so each load takes 64 contiguous bytes of a row from its
-// four lanes; without, k = 8 lg .. 8 lg + 7.  B is stored to match.
+// live(g) as for the FP32 core's loaders.  A step is 32 k.  row(m, lg): the
+// address part of one output row for lane group lg; issue: starts a lane's
+// loads; resolve: its 8 values.  Addresses along k are kbase(k0), of the step
+// from k0 (wave-uniform; K a multiple of 32), or with TABLE offset(k), of one k
+// (any K); both take any k and past K make every address out of range, so that
+// such elements read zero.  With PERM lane group lg holds k = 4 lg .. 4 lg + 3
+// and 16 + 4 lg .. of the step, so each load takes 64 contiguous bytes of a row
+// from its four lanes; without, k = 8 lg .. 8 lg + 7.  B is stored to match.
 
 // ---------------------------------------------------------- B operands ---
 //
@@ -148,9 +149,8 @@ struct SbCol {
 // ----------------------------------------------------------- epilogues ---
 //
 // A lane stores FN consecutive columns of a row at once; n is a multiple of
-// FN and so are the output's columns and row pitch.  v = alpha*acc (+ bias)
-// (relu) (* [mask > 0]) (+ beta*old), the mask and the old value read only
-// where there is one.
+// FN and so are the output's columns and row pitch.  v = alpha*acc (* [mask > 0])
+// (+ beta*old), the mask and the old value read only where there is one.
 template <int N>
 using FVec = float __attribute__((ext_vector_type(N)));
 
@@ -174,51 +174,11 @@ __device__ __forceinline__ FVec<FN> row_of(const f32x4 (&a)[FN], int r) {
   return v;
 }
 
-// One row-major block C[g](m, n).
-struct SeStore {
-  int M = 0, N = 0;
-  float* C[kMaxGroups] = {};
-  long ldc = 0;
-  float alpha = 1.f, beta = 0.f;
-  const float* bias[kMaxGroups] = {};
-  int relu = 0;
-  const float* mask[kMaxGroups] = {};
-  float* sums[kMaxGroups] = {};  // the column sums of B (a bias gradient), += beta * old
-
-  __device__ __forceinline__ void store_sum(int g, int n, float t) const {
-    float* d = sums[g] + n;
-    *d = beta != 0.f ? t + beta * *d : t;
-  }
-
-  struct Params {
-    float* c;
-    const float* b;
-    const float* mk;
-    int M, N, ldc;
-    float alpha, beta;
-    int relu;
-  };
-  struct Bound {
-    Params q;
-    __amdgpu_buffer_rsrc_t rc, rb, rm;
-    __device__ __forceinline__ uint32_t off(int m, int n) const {
-      return m < q.M && n < q.N ? (uint32_t(m) * uint32_t(q.ldc) + uint32_t(n)) * 4u : kBad;
-    }
-    template <int FN>
-    __device__ __forceinline__ FVec<FN> bias(int n) const { return ld_vec<FN>(rb, uint32_t(n) * 4u); }
-    __device__ __forceinline__ float alpha() const { return q.alpha; }
-    __device__ __forceinline__ float beta() const { return q.beta; }
-    __device__ __forceinline__ bool relu() const { return q.relu != 0; }
-    __device__ __forceinline__ bool masked() const { return q.mk != nullptr; }
-    __device__ __forceinline__ bool accumulates() const { return q.beta != 0.f; }
-  };
+// No epilogue: partials of K, which their reader sums.
+struct SePartials {
+  static constexpr bool PARTIALS = true;
+  int M = 0;
   __device__ __forceinline__ int rows(int) const { return M; }
-  __device__ __forceinline__ Bound bind(int g) const {
-    const Params q = pin_pod(Params{C[g], bias[g], mask[g], M, N, int(ldc), alpha, beta, relu});
-    const uint32_t bytes = q.M > 0 ? uint32_t((q.M - 1) * q.ldc + q.N) * 4u : 0u;
-    return Bound{q, make_res(q.c, bytes), make_res(q.b, q.b ? uint32_t(q.N) * 4u : 0u),
-                 make_res(q.mk, q.mk ? bytes : 0u)};
-  }
 };
 
 // ------------------------------------------------------------ the core ---
@@ -509,8 +469,10 @@ __global__ __launch_bounds__(64 * NW) void k_split(LA la, LB lb, EP ep, float* w
     }
   }
 
-  const int n = n0 + FN * lr, prows = M + ones;  // a partial's rows: the column sums below the product
-  if constexpr (VB::COL) {
+  const int n = n0 + FN * lr;
+  if constexpr (EP::PARTIALS) {
+    const int prows = M + ones;  // a partial's rows: the column sums below the product
+    float* const part = ws + (long(g) * splits + split) * prows * N;
     if (ones && blockIdx.x == 0) {
       float* red = reinterpret_cast<float*>(lds);  // the loop ended with a barrier
       bs.put_sums(red, tid);
@@ -519,14 +481,10 @@ __global__ __launch_bounds__(64 * NW) void k_split(LA la, LB lb, EP ep, float* w
         float t = 0.f;
 #pragma unroll
         for (int q = 0; q < KB / 4; ++q) t += red[q * BN + tid];
-        if (splits > 1) ws[((long(g) * splits + split) * prows + M) * N + n0 + tid] = t;
-        else ep.store_sum(g, n0 + tid, t);
+        part[long(M) * N + n0 + tid] = t;
       }
     }
-  }
-  if (splits > 1) {
-    const __amdgpu_buffer_rsrc_t rw =
-        make_res(ws + (long(g) * splits + split) * prows * N, uint32_t(M) * uint32_t(N) * 4u);
+    const __amdgpu_buffer_rsrc_t rw = make_res(part, uint32_t(M) * uint32_t(N) * 4u);
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -534,33 +492,31 @@ __global__ __launch_bounds__(64 * NW) void k_split(LA la, LB lb, EP ep, float* w
         const int m = mw + i * 16 + 4 * lg + r;
         st_vec(rw, m < M && n < N ? (uint32_t(m) * uint32_t(N) + uint32_t(n)) * 4u : kBad, row_of<FN>(acc[i], r));
       }
-    return;
-  }
-  const auto eb = ep.bind(g);
-  const auto bias = eb.template bias<FN>(n);
+  } else {
+    const auto eb = ep.bind(g);
 #pragma unroll
-  for (int i = 0; i < WM; ++i) {
-    uint32_t off[4];
-    FVec<FN> keep[4], old[4];
+    for (int i = 0; i < WM; ++i) {
+      uint32_t off[4];
+      FVec<FN> keep[4], old[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) off[r] = eb.off(mw + i * 16 + 4 * lg + r, n);
-    if (eb.masked())
+      for (int r = 0; r < 4; ++r) off[r] = eb.off(mw + i * 16 + 4 * lg + r, n);
+      if (eb.masked())
 #pragma unroll
-      for (int r = 0; r < 4; ++r) keep[r] = ld_vec<FN>(eb.rm, off[r]);
-    if (eb.accumulates())
+        for (int r = 0; r < 4; ++r) keep[r] = ld_vec<FN>(eb.rm, off[r]);
+      if (eb.accumulates())
 #pragma unroll
-      for (int r = 0; r < 4; ++r) old[r] = ld_vec<FN>(eb.rc, off[r]);
+        for (int r = 0; r < 4; ++r) old[r] = ld_vec<FN>(eb.rc, off[r]);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      FVec<FN> v = row_of<FN>(acc[i], r);
+      for (int r = 0; r < 4; ++r) {
+        FVec<FN> v = row_of<FN>(acc[i], r);
 #pragma unroll
-      for (int j = 0; j < FN; ++j) {
-        v[j] = eb.alpha() * v[j] + bias[j];
-        if (eb.relu()) v[j] = v[j] > 0.f ? v[j] : 0.f;
-        if (eb.masked() && !(keep[r][j] > 0.f)) v[j] = 0.f;
-        if (eb.accumulates()) v[j] += eb.beta() * old[r][j];
+        for (int j = 0; j < FN; ++j) {
+          v[j] *= eb.alpha();
+          if (eb.masked() && !(keep[r][j] > 0.f)) v[j] = 0.f;
+          if (eb.accumulates()) v[j] += eb.beta() * old[r][j];
+        }
+        st_vec(eb.rc, off[r], v);
       }
-      st_vec(eb.rc, off[r], v);
     }
   }
 }
@@ -578,23 +534,30 @@ struct SplitTile {
 SplitTile split_tile(long M, long N, long groups);
 long split_tiles(long M, long N, long groups);  // its 64 x 64 tiles, those of 32 columns counted half
 
-// splits > 1: partials [groups][splits][M + ones][N] to ws.
+template <int WM, int FN, class LA, class LB, class EP>
+inline int launch_split(ttrl_ctx* ctx, const LA& la, const LB& lb, const EP& ep, int M, int N, int K, int groups,
+                        const char* name, int ones, float* ws, int splits, int kchunk) {
+  constexpr int NW = 4;
+  const dim3 grid(ceil_div(M, NW * WM * 16), ceil_div(N, FN * 16), unsigned(groups * splits));
+  hipLaunchKernelGGL((k_split<WM, FN, NW, LA, LB, EP>), grid, dim3(64 * NW), 0, stream_of(ctx), la, lb, ep, ws, M, N, K,
+                     kchunk, splits, ones);
+  return check_launch(name);
+}
+
 template <class LA, class LB, class EP>
-inline int run_split(ttrl_ctx* ctx, const SplitTile& t, const LA& la, const LB& lb, const EP& ep, int M, int N, int K,
-                     int groups, const char* name, int ones = 0, float* ws = nullptr, int splits = 1, int kchunk = 0) {
-  if (splits == 1) kchunk = int(ceil_div(K, kSplitKB)) * kSplitKB;
+inline int run_split(ttrl_ctx* ctx, const LA& la, const LB& lb, const EP& ep, int M, int N, int K, int groups,
+                     const char* name) {
+  const SplitTile t = split_tile(M, N, groups);
+  const int kchunk = int(ceil_div(K, kSplitKB)) * kSplitKB;
   auto go = [&](auto wm, auto fn) {
-    constexpr int WM = decltype(wm)::value, FN = decltype(fn)::value, NW = 4;
-    const dim3 grid(ceil_div(M, NW * WM * 16), ceil_div(N, FN * 16), unsigned(groups * splits));
-    hipLaunchKernelGGL((k_split<WM, FN, NW, LA, LB, EP>), grid, dim3(64 * NW), 0, stream_of(ctx), la, lb, ep, ws, M, N,
-                       K, kchunk, splits, ones);
+    return launch_split<decltype(wm)::value, decltype(fn)::value>(ctx, la, lb, ep, M, N, K, groups, name, 0, nullptr, 1,
+                                                                  kchunk);
   };
   using I1 = std::integral_constant<int, 1>;
   using I2 = std::integral_constant<int, 2>;
   using I4 = std::integral_constant<int, 4>;
-  if (t.fn == 4) t.wm == 2 ? go(I2{}, I4{}) : go(I1{}, I4{});
-  else t.wm == 2 ? go(I2{}, I2{}) : go(I1{}, I2{});
-  return check_launch(name);
+  if (t.fn == 4) return t.wm == 2 ? go(I2{}, I4{}) : go(I1{}, I4{});
+  return t.wm == 2 ? go(I2{}, I2{}) : go(I1{}, I2{});
 }
 
 }  // namespace ttrl
