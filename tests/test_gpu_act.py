@@ -404,3 +404,24 @@ def test_q_act_weights_staged_in_rounds(device, B, K, A):
     got = q.numpy()
     assert np.all(np.abs(got - want) <= bound)
     assert np.array_equal(act.numpy(), np.argmax(got, 1))
+
+
+@pytest.mark.parametrize("K", [64, 255, 256, 300, 513])
+@pytest.mark.parametrize("A", [6, 9, 15, 16, 18, 24, 32])
+def test_q_act_rows_do_not_depend_on_the_batch(device, K, A):
+    """A row's sums are the same bits whether its weights are read directly or
+    through LDS, which the batch, the width and K decide."""
+    from ttrl_amd.engine.tensor import DeviceArray
+
+    rng = np.random.default_rng(K + A)
+    h, W = rng.standard_normal((9, K)).astype(np.float32), rng.standard_normal((K, A)).astype(np.float32)
+    dW = DeviceArray(device, (K, A))
+    dW.upload(W)
+    out = {}
+    for B in (1, 2, 3, 4, 9):
+        dh, q, act = DeviceArray(device, (B, K)), DeviceArray(device, (B, A)), DeviceArray(device, (B,), np.int32)
+        dh.upload(np.ascontiguousarray(h[:B]))
+        device.call("ttrl_q_act", B, K, A, dh.ptr, dW.ptr, None, q.ptr, act.ptr)
+        out[B] = q.numpy()
+    for B in (1, 2, 3, 4):
+        assert np.array_equal(out[B], out[9][:B]), B
