@@ -18,11 +18,8 @@
 // each column are combined by an xor butterfly, which leaves the identical
 // total in every lane, so any lane can take the decision.  The layer is tiny
 // (K <= a few thousand, N <= 32): latency, not bandwidth or MFMA, bounds it.
-// Wide heads (N > 8) of more than one row take the weights through LDS: a
-// lane reading its own weight rows touches a cache line per lane and element
-// (K 300, N 16: 4 rows 13.4 us, 1,000 rows 14.2; staged 9.9 and 10.8).  One
-// row alone waits longer for the staging than for its own reads (9.0 / 10.1),
-// and so does a narrow head at any batch (K 512, N 6: 5.2 to 6.1 / 6.5 to 7.7).
+// Wide heads of more than one row may take the weights through LDS (staged):
+// a lane reading its own weight rows touches a cache line per lane and element.
 #include "common.hpp"
 
 #include <cmath>
@@ -72,9 +69,9 @@ __global__ __launch_bounds__(kActThreads) void k_head_act(ActArgs a) {
   __shared__ float wt[STAGED ? kActCols * (NP + 1) : 1];  // odd pitch: a column's 64 lanes hit 64 banks
   const int tid = threadIdx.x, lane = tid & 63;
   const int row = blockIdx.x * kActRows + (tid >> 6), b = min(row, a.B - 1);
-  // A wavefront past the last row leaves; in the staged form it first helps to
-  // stage (its reads beside the row's own would make one row of 16 columns over
-  // K 512 take 18.3 us instead of 9.6).
+  // A wavefront past the last row leaves, in the staged form after it has helped
+  // to stage (left to read weights beside the row's own, three of them made one
+  // row of 16 columns over K 512 take 18.3 us instead of 9.5).
   if (!STAGED && row >= a.B) return;
   const int N = a.N, n1 = a.n1, n2 = a.N - a.n1;
   const float* hb = a.h + long(b) * a.K;
@@ -232,12 +229,31 @@ __global__ __launch_bounds__(kActThreads) void k_head_act(ActArgs a) {
   }
 }
 
+// Whether a head of N columns stages its weights, timed over K 64 to 1,024, 9 to
+// 32 columns, 1 to 1,024 rows, both modes (us, direct reads / staged; greedy
+// unless said).  A single row waits longer for the staging than for its own
+// reads, and so does a narrow head at any batch (K 512, N 6: 5.2 to 6.1 / 6.5 to
+// 7.7).  K under one round of kActCols leaves the direct reads no whole round to
+// keep in flight: staged (K 128, 8 rows: N 9 7.1 / 6.6, N 16 8.5 / 7.1).  Beyond,
+// under 16 columns several lanes share a line and direct reads win (K 512, 8
+// rows: N 9 10.2 / 10.9, N 14 11.7 / 12.4); from 16 each has its own, and rows
+// that share the staged weights win (K 512, 8 rows: N 16 19.4 / 13.2, N 18 22.2 /
+// 19.9, N 32 36.2 / 24.5).  Two rows: N 18 20.1 / 19.1 but N 16 12.2 / 12.6, N 28
+// 18.6 / 22.1, N 32 22.4 / 23.5; squashed, whose two matrices split a line, N 16
+// 12.0 / 11.6, N 32 21.6 / 19.8.
+bool staged_pays(ActMode mode, int rows, int K, int N) {
+  if (rows < 2 || N <= 8) return false;
+  if (K < kActCols) return true;
+  if (N < 16) return false;
+  return rows > 2 || mode == ActMode::Squashed || (N > 16 && N <= 20);
+}
+
 template <ActMode MODE>
 int launch_head_act(ttrl_ctx* ctx, ActArgs a, int width, const char* name) {
   a.d1.set(a.n1);
   a.d2.set(a.N > a.n1 ? a.N - a.n1 : 1);
   const dim3 grid(unsigned((a.B + kActRows - 1) / kActRows)), block(kActThreads);
-  const bool staged = a.B > 1;
+  const bool staged = staged_pays(MODE, a.B, a.K, width);
   if (width <= 8) hipLaunchKernelGGL((k_head_act<MODE, 8, false>), grid, block, 0, stream_of(ctx), a);
   else if (width <= 16 && staged) hipLaunchKernelGGL((k_head_act<MODE, 16, true>), grid, block, 0, stream_of(ctx), a);
   else if (width <= 16) hipLaunchKernelGGL((k_head_act<MODE, 16, false>), grid, block, 0, stream_of(ctx), a);
