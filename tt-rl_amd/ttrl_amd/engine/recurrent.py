@@ -32,11 +32,29 @@ from ttrl_amd.engine.tensor import DeviceArray
 __all__ = ["GATES", "GRU", "GRUCell"]
 
 GATES = ("reset", "update", "candidate")
-# Workgroups (8 units x 8 sequences each) up to which a ragged step runs in one
-# launch: past two to three a CU the GEMM's larger tiles read less.  Forward
-# and backward of 8 steps: H 515, 64 sequences (520) 307 -> 279 us, 128 (1040)
-# 374 -> 420; H 250, 128 sequences (512) 264 -> 186.
+# A ragged step (8 units x 8 sequences a workgroup) runs in one launch while
+# either its sequences are one row of workgroups, which read W_hh once, or the
+# W_hh that all rows read fits the L2s of the eight XCDs (4 MiB each) closely
+# and the workgroups are few; past that the GEMM's larger tiles read less.
+# Forward and backward of 8 steps, two launches a step / one, us: H 515, 96
+# sequences (38 MB) 351 / 348; H 630, 64 (38 MB) 357 / 348; H 777, 40 (36 MB) 349 / 316,
+# 48 (43 MB) 360 / 387; H 1001, 24 (36 MB) 355 / 348, 32 (48 MB) 374 / 391; H 1300,
+# 8 sequences 309 / 258, 9 (41 MB) 311 / 389; H 2050, 8 663 / 624, 16 718 / 992.
+_RAGGED_BYTES = 38_500_000
 _RAGGED_GROUPS = 640
+
+
+def _step_kernel(H: int, B: int, aligned: bool, two_launch: bool) -> str | None:
+    """Which one-launch step B sequences of H units take: "fused" (its own
+    layout: H a multiple of 16, float4-aligned operands), "ragged", or None for
+    a GEMM and a cell kernel per step."""
+    if H > 8192:
+        return None
+    if H % 16 == 0 and aligned:
+        return "fused"
+    rows = -(-B // 8)
+    few = -(-H // 8) * rows <= _RAGGED_GROUPS
+    return "ragged" if few and not two_launch and (rows == 1 or 12 * H * H * rows <= _RAGGED_BYTES) else None
 
 
 class GRUCell(Module):
@@ -139,11 +157,7 @@ def unroll(cell: GRUCell, x: Tensor, h0: Tensor, done: Tensor | None):
         return arr.view(t * B * width, (B, width))
 
     W_hh = cell.weight_hh.data
-    # One launch per step, else a GEMM and a cell kernel per step.  Off the
-    # fused kernels' own layout (H a multiple of 16, float4-aligned operands)
-    # the ragged form while its workgroups are few.
-    step = "fused" if H % 16 == 0 and all(a.ptr % 16 == 0 for a in (HIN, W_hh)) else "ragged"
-    fused = H <= 8192 and (step == "fused" or (-(-H // 8) * -(-B // 8) <= _RAGGED_GROUPS and not cell.two_launch_steps))
+    step = _step_kernel(H, B, all(a.ptr % 16 == 0 for a in (HIN, W_hh)), cell.two_launch_steps)
     _linear(dev, X, cell.weight_ih, cell.bias_ih, GI, T * B, F, G)
     dev.call("ttrl_gru_mask", B, H, h0.data.vp, done_at(0), HIN.vp)
     for t in range(T):
@@ -151,7 +165,7 @@ def unroll(cell: GRUCell, x: Tensor, h0: Tensor, done: Tensor | None):
         last = t + 1 == T
         done_next = None if last else done_at(t + 1)
         hin_next = None if last else at(HIN, t + 1, H).vp
-        if fused:
+        if step:
             dev.call("ttrl_gru_step_" + step, B, H, gi.vp, hin.vp, W_hh.vp, cell.bias_hh.data.vp, gh.vp, out.vp,
                      done_next, hin_next)
         else:
@@ -185,7 +199,7 @@ def unroll(cell: GRUCell, x: Tensor, h0: Tensor, done: Tensor | None):
         DGI = DeviceArray(dev, (T, B, G))
         DGH = DeviceArray(dev, (T, B, G))
         need_h0 = h0.requires_grad
-        if fused:
+        if step:
             dhin0 = _backward_fused(grad, DGI, DGH, need_h0)
         else:
             dhin0 = _backward_steps(grad, DGI, DGH, need_h0)
