@@ -121,7 +121,8 @@ def test_conv_backward_choice_gives_the_separate_gradients(device, B):
 
     Cin, H, O, k, s = 32, 20, 64, 4, 2
     OH = (H - k) // s + 1
-    g = _lib.ConvGeom(B, Cin, H, H, O, k, s, 0, _lib.LAYOUT_NHWC_F32)
+    # the choice between launches of the FP32 core, at 256 too
+    g = _lib.ConvGeom(B, Cin, H, H, O, k, s, 0, _lib.LAYOUT_NHWC_F32 | _lib.CONV_FP32_ORDER)
     rng = np.random.default_rng(B)
     x = rng.standard_normal((B, H, H, Cin)).astype(np.float32)
     dy = rng.standard_normal((B, OH, OH, O)).astype(np.float32)
@@ -142,4 +143,5 @@ def test_conv_backward_choice_gives_the_separate_gradients(device, B):
     assert _rel(dw2.numpy() - 0.5, 2 * dw.numpy()) < 1e-5
     assert _rel(db2.numpy() - 0.5, 2 * db.numpy()) < 1e-5
     assert _rel(dx2.numpy() - 0.5, 2 * dx.numpy()) < 1e-5
-    assert f"ttrl_conv2d_backward:pair|" in device.export_plans()
+    key = f"ttrl_conv2d_backward:pair|0|{B}|{Cin}|{H}|{H}|{O}|{k}|{k}|{s}|0|{(B * OH * OH * O + 63) // 64 * 64}|1|0"
+    assert any(row.endswith("\t" + key) for row in device.export_plans().splitlines())

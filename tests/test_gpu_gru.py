@@ -234,3 +234,64 @@ def test_ragged_steps_match_float64(device, B, H):
     for got, want in ((dhin, dhin64), (dgi_o, np.concatenate([drp, dzp, dcp], 1)),
                       (dgh_o, np.concatenate([drp, dzp, dcp * r], 1)), (dhz_o, dh * z)):
         assert _rel(got.numpy()[ok], want[ok]) < 1e-5
+
+
+@pytest.mark.parametrize("H", [250, 100])
+def test_two_launch_steps_keep_their_bits(device, monkeypatch, H):
+    """A cell with two_launch_steps unrolls by a GEMM and a cell kernel per
+    step, forward and backward, as every cell off the 16s does past the
+    one-launch step's range; without it the one-launch sums differ in their last
+    bits."""
+    from ttrl_amd.engine import recurrent
+    from ttrl_amd.engine.autograd import Tensor
+    from ttrl_amd.engine.tensor import DeviceArray
+
+    T, B, F = 5, 24, 33
+    np.random.seed(H)
+    gru = recurrent.GRU(F, H, device)
+    rng = np.random.default_rng(H)
+    x = rng.standard_normal((T, B, F)).astype(np.float32)
+    h0 = rng.standard_normal((B, H)).astype(np.float32)
+    done = (rng.random((T, B, 1)) < 0.2).astype(np.float32)
+    G = _arr(device, rng.standard_normal((T, B, H)))
+
+    def run():
+        xt, ht = (Tensor.from_numpy(v, device, requires_grad=True) for v in (x, h0))
+        for p in gru.parameters():
+            p.grad = None
+        outs, _ = gru(xt, ht, Tensor.from_numpy(done, device))
+        seed = DeviceArray(device, (T, B, H))
+        seed.copy_from(G)
+        outs.grad, outs._grad_owned = seed, True
+        outs._backward(seed)
+        return [outs.numpy(), xt.grad.numpy(), ht.grad.numpy()] + [p.grad.numpy() for p in gru.parameters()]
+
+    one = run()
+    gru.cell.two_launch_steps = True
+    two = run()
+    gru.cell.two_launch_steps = False
+    monkeypatch.setattr(recurrent, "_RAGGED_GROUPS", 0)
+    past = run()
+    assert all(np.array_equal(a, b) for a, b in zip(two, past))
+    assert not np.array_equal(one[0], two[0])
+
+
+def test_ppo_learners_keep_their_summation_order(device):
+    """Every convolution of a PPO learner stays on the FP32 core, and a
+    recurrent one's GRU on two launches off the 16s."""
+    from ttrl_amd.algos.ppo import PPOConfig, PPOLearner, RecurrentConfig, RecurrentPPOLearner
+    from ttrl_amd.engine.conv import Conv2d
+    from ttrl_amd.engine.recurrent import GRUCell
+    from ttrl_amd.nets.acting import _walk_modules
+    from ttrl_amd.spaces import ActionSpec, ObsSpec
+
+    obs, act = ObsSpec.image((4, 36, 36)), ActionSpec.discrete(6)
+    for learner in (PPOLearner(obs, act, device, cfg=PPOConfig(minibatch_size=32, n_steps=16), seed=0),
+                    RecurrentPPOLearner(obs, act, device, seed=0, cfg=PPOConfig(
+                        minibatch_size=32, n_steps=16, recurrent=RecurrentConfig(hidden_size=100, seq_len=8)))):
+        mods = [m for _, m in _walk_modules(learner.net)]
+        convs = [m for m in mods if isinstance(m, Conv2d)]
+        cells = [m for m in mods if isinstance(m, GRUCell)]
+        assert convs and all(m.fp32_order for m in convs)
+        assert bool(cells) == isinstance(learner, RecurrentPPOLearner) and all(m.two_launch_steps for m in cells)
+        learner.close()

@@ -252,6 +252,70 @@ def test_both_gradients_choose_their_cores_apart(dev, dims, dw, dx, bank):
     assert separate or not (dw and dx)  # both well past the lines
 
 
+@pytest.mark.parametrize("dims", [(62, 4, 84, 32, 8, 4, True), (256, 32, 20, 64, 4, 2), (128, 64, 9, 64, 3, 1)])
+def test_the_flag_gives_the_fp32_core(dev, dims):
+    """Output gradients one float off 16-byte alignment keep any layer on the
+    FP32 core, by the same plan: TTRL_CONV_FP32_ORDER gives its bits."""
+    from ttrl_amd.engine.tensor import to_device
+
+    layer = _Layer(dev, *dims)
+    want = layer.weight(True), None if layer.dims[6] else layer.input(True)
+    dy = layer.dy.numpy()
+    layer.dy = to_device(np.concatenate([[np.float32(0.0)], dy.ravel()]), dev).view(1, dy.shape)
+    assert np.array_equal(layer.weight(False), want[0])
+    if want[1] is not None:
+        assert np.array_equal(layer.input(False), want[1])
+
+
+# Output gradients masked by the layer's own ReLU (a copy in the workspace, the
+# partials below it), outputs added to, kernels whose classes take several
+# launches (stride 3: nine), and padding (the weight gradient then on the FP32
+# core): (batch, channels, size, out, kernel, stride, padding).
+FORMS = [(256, 32, 20, 64, 4, 2, 0), (128, 64, 9, 64, 3, 1, 0), (400, 32, 15, 64, 3, 3, 0), (400, 24, 13, 32, 5, 4, 0),
+         (64, 32, 20, 64, 3, 1, 1), (300, 20, 12, 32, 4, 2, 1)]
+
+
+@pytest.mark.parametrize("b,c,size,o,k,s,p", FORMS)
+@pytest.mark.parametrize("entry", ["both", "apart", "deferred"])
+def test_masks_sums_strides_and_padding(dev, b, c, size, o, k, s, p, entry):
+    from ttrl_amd import _lib
+    from ttrl_amd.engine.tensor import DeviceArray, to_device
+
+    rng = np.random.default_rng(b + size)
+    x = rng.standard_normal((b, size, size, c)).astype(np.float32)
+    xp = np.pad(x, ((0, 0), (p, p), (p, p), (0, 0)))
+    a = _patches(xp, k, s)
+    wt = rng.standard_normal((k * k * c, o)).astype(np.float32)
+    dy, y = (rng.standard_normal((a.shape[0], o)).astype(np.float32) for _ in range(2))
+    geom = C.byref(_lib.ConvGeom(b, c, size, size, o, k, s, p, _lib.LAYOUT_NHWC_F32))
+    xd, dyd, yd, wd = (to_device(v, dev) for v in (x, dy, y, wt))
+    dw, db, dx = DeviceArray(dev, wt.shape), DeviceArray(dev, (1, o)), DeviceArray(dev, x.shape)
+    for out in (dw, db, dx):
+        out.fill(3.0)
+    beta = np.float32(0.0 if entry == "deferred" else 0.5)  # the deferred weight gradient is written fresh
+    half = C.c_float(0.5)
+    if entry == "both":
+        dev.call("ttrl_conv2d_backward", geom, xd.vp, half, dyd.vp, yd.vp, wd.vp, dw.vp, db.vp, half, dx.vp, xd.vp, half)
+    elif entry == "apart":
+        dev.call("ttrl_conv2d_backward_weight", geom, xd.vp, half, dyd.vp, yd.vp, dw.vp, db.vp, half)
+        dev.call("ttrl_conv2d_backward_input", geom, dyd.vp, yd.vp, wd.vp, dx.vp, xd.vp, half, half)
+    else:
+        src = _lib.GradSource()
+        dev.call("ttrl_conv2d_backward_deferred", geom, xd.vp, half, dyd.vp, yd.vp, wd.vp, dw.vp, db.vp, dx.vp, xd.vp,
+                 half, 3, C.byref(src))
+        if src.kind != _lib.GRAD_NONE:
+            dev.call("ttrl_grad_sources_materialize", 1, C.byref(src))
+    g = np.where(y > 0, dy, np.float32(0.0)).astype(np.float64)
+    w64 = wt.astype(np.float64)
+    crop = (slice(None), slice(p, p + size), slice(p, p + size))
+    dx64, mag = (_scatter(f(g) @ f(w64).T, xp.shape, k, s)[crop] for f in (lambda v: v, np.abs))
+    # the float32 epilogue rounds twice more, on the old value among them
+    for got, want, terms, m in ((dw, 0.5 * (a.T @ g) + beta * 3.0, a.shape[0], np.abs(a).T @ np.abs(g) + 6.0),
+                                (db, g.sum(0)[None] + beta * 3.0, a.shape[0], np.abs(g).sum(0)[None] + 6.0),
+                                (dx, np.where(x > 0, 0.5 * dx64, 0.0) + 1.5, k * k * o, mag + 6.0)):
+        assert np.all(np.abs(got.numpy() - want) <= _bound(terms, m))
+
+
 def test_short_sums_of_the_worst_operands(dev):
     """Sums of 32 products (one step of the core) of operands whose mantissa
     leaves most in the lower parts (0x00ffff).  In 2^-24 of the sum: 1 for the
