@@ -244,14 +244,17 @@ int ttrl_linear_backward(ttrl_ctx* ctx, const ttrl_linear_desc* desc);
 
 #define TTRL_LAYOUT_NHWC_F32 0 /* [B][H][W][C] fp32 activations */
 #define TTRL_LAYOUT_NCHW_U8 1  /* [B][C][H][W] uint8 frames */
-/* Or-ed into in_layout: gradients summed by the FP32 matrix core alone, for
- * callers whose next step turns a last-bit difference into a decision. */
+/* A flag beside the layout, or-ed into in_layout: the gradient entry points sum
+ * on the FP32 matrix core alone, whatever the size, for callers whose next step
+ * turns a last-bit difference into a decision.  Without it large gradients are
+ * summed on the bf16 matrix cores from operands split in three, closer to
+ * float64 in another order.  Forward calls take no notice of it. */
 #define TTRL_CONV_FP32_ORDER 16
 
 /* Geometry of ConvGeometry (ttrl/engine/conv/geometry.py:94-199), square kernel. */
 typedef struct ttrl_conv_geom {
   int batch, in_c, in_h, in_w, out_c, kernel, stride, padding;
-  int in_layout;
+  int in_layout; /* TTRL_LAYOUT_*, TTRL_CONV_FP32_ORDER or-ed in or not */
 } ttrl_conv_geom;
 
 /* (size + 2p - k)/s + 1, refusing ragged geometry (ttrl/engine/conv/geometry.py:107-119). */
@@ -284,9 +287,10 @@ int ttrl_conv2d_backward_input(ttrl_ctx* ctx, const ttrl_conv_geom* geom, const 
 /* Both gradients of one conv2d node's backward (ttrl/engine/conv/backward.py:33-78):
  * ttrl_conv2d_backward_weight(x, x_scale, dy, ymask, dwt, db, beta_w) and
  * ttrl_conv2d_backward_input(dy, ymask, wt, dx, xmask, x_scale, beta_x), the
- * two GEMMs sharing one launch or as two launches with their own tile shapes,
- * whichever the context measured faster for the geometry on its first call
- * outside capture (kept with the context's GEMM plans).  fp32 NHWC inputs
+ * two GEMMs sharing one launch or as separate launches, each with its own tile
+ * shape and on the core its own entry point takes, whichever the context
+ * measured faster for the geometry on its first call outside capture (kept with
+ * the context's GEMM plans).  fp32 NHWC inputs
  * only (a uint8 frame input has no gradient); db may be NULL. */
 int ttrl_conv2d_backward(ttrl_ctx* ctx, const ttrl_conv_geom* geom, const void* x, float x_scale, const float* dy,
                          const float* ymask, const float* wt, float* dwt, float* db, float beta_w, float* dx,

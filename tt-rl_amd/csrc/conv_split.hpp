@@ -164,8 +164,11 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 //     launch: the second layer's partials at 5,184 pixels (170 M) 9.6 / 8.6, the
 //     third's at 4,704 (173 M) 9.6 / 8.7.  Of bytes (updates of a DQN, 24 to 100
 //     images of 52 to 84): at 59 M 122 / 120, at 67 M 112.3 / 111, at 88 M 128 / 124,
-//     at 105 M equal, the optimizer step reading twice the parts; at 21 M 84 / 87, at
-//     28 M 86 / 88.
+//     at 105 M 133.2 / 132.1 (its launch 9.2 / 8.1, the optimizer step, which reads
+//     twice the parts, 15.1 / 15.6); at 21 M 84 / 87, at 28 M 86 / 88.
+// Twice the parts added one after another show where all products have one sign
+// (error against float64 1.1e-7 to 1.3e-7, FP32 core 0.7e-7 to 1.5e-7); sums of
+// either sign are the closer by 1.1 to 3 times.
 constexpr int kMaxDwSplits = 64;
 constexpr long kSplitProducts = 200'000'000, kSplitBank = 150'000'000, kSplitBankU8 = 40'000'000;
 constexpr long kSplitArea = 8192, kSplitAreaU8 = 6144;

@@ -20,8 +20,8 @@
 // main sum is rounded once per 32 k: weight gradients at batch 1024 6.9e-7 ->
 // 2.2e-7, input gradients 2.7e-7 -> 8.5e-8, at K = 32 (2 x 2 kernels, stride 2)
 // 1.0e-7 -> 3.9e-8.  What bounds it: a stage's chain of loads, splits (5.5 VALU
-// instructions per float) and LDS round trips; the matrix core is busy about a
-// third of the time.
+// instructions per float) and LDS round trips; the matrix core is busy 10 to 12 %
+// of the time at batch 256, 23 % at 1024.
 //
 // One workgroup owns BM x BN of the output, NW wavefronts along M, each
 // WM x FN fragments of 16 x 16.
