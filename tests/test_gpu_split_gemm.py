@@ -299,6 +299,11 @@ def test_masks_sums_strides_and_padding(dev, b, c, size, o, k, s, p, entry):
     elif entry == "apart":
         dev.call("ttrl_conv2d_backward_weight", geom, xd.vp, half, dyd.vp, yd.vp, dw.vp, db.vp, half)
         dev.call("ttrl_conv2d_backward_input", geom, dyd.vp, yd.vp, wd.vp, dx.vp, xd.vp, half, half)
+        other = DeviceArray(dev, x.shape)
+        other.fill(3.0)
+        fp32 = C.byref(_lib.ConvGeom(b, c, size, size, o, k, s, p, _lib.LAYOUT_NHWC_F32 | _lib.CONV_FP32_ORDER))
+        dev.call("ttrl_conv2d_backward_input", fp32, dyd.vp, yd.vp, wd.vp, other.vp, xd.vp, half, half)
+        assert not np.array_equal(dx.numpy(), other.numpy())  # every form is the split core's
     else:
         src = _lib.GradSource()
         dev.call("ttrl_conv2d_backward_deferred", geom, xd.vp, half, dyd.vp, yd.vp, wd.vp, dw.vp, db.vp, dx.vp, xd.vp,
